@@ -175,10 +175,12 @@ def _inputs(case, seed):
 
 
 class _View:
-    """Device memory of the library's as the array interface that torch reads."""
+    """Device memory of the library's as the array interface that torch reads. A tensor made from it holds it, and it
+    holds the memory's owner."""
 
-    def __init__(self, ptr, halves):
-        self.__cuda_array_interface__ = dict(shape=(halves,), typestr="<f2", data=(ptr, False), version=2)
+    def __init__(self, buf, halves):
+        self.owner = buf
+        self.__cuda_array_interface__ = dict(shape=(halves,), typestr="<f2", data=(buf.data_ptr(), False), version=2)
 
 
 def prepare(case, seed):
@@ -248,7 +250,7 @@ def run(s):
         # a new prompt's context replaces the last one's
         s["context"] = s["dit"].cache_context(s["ctx"])
         halves = kiln_amd.kv_prepped_bytes(case["real"], HEADS) // 2
-        return [torch.as_tensor(_View(s["context"].kv(i).data_ptr(), halves), device=DEV) for i in range(BLOCKS)]
+        return [torch.as_tensor(_View(s["context"].kv(i), halves), device=DEV) for i in range(BLOCKS)]
     return s["dit"].forward(s["outs"], s["latent"], 0.5, s["ctxs"], nag=s["nagc"])
 
 
