@@ -23,25 +23,19 @@
 //    chunks, chunk c of row r at position c ^ ((r >> 1) & 3): the DMA reads whole row segments (coalesced)
 //    and the MFMA operand reads (16 rows x one chunk per 16 lanes) are bank-conflict free.
 //  * the operands of k tile t+1 are read from LDS while the MFMAs of k tile t run.
+//  * products too small to fill the chip with these tiles run on gemm16s.hip's.
 //  * 1-D grid, XCD-aware: workgroup b runs on XCD b % 8, and each XCD takes a contiguous range of tiles in
 //    groups of 4 row tiles, so the workgroups resident on one XCD share A and W tiles in its L2.
-#include <type_traits>
-
-#include "common.hpp"
-#include "internal.hpp"
+#include "gemm16.hpp"
 
 namespace kiln {
 
-
-constexpr int GBN = 256;             // weight rows (n) per workgroup
-constexpr int GBK = 32;              // k per tile: one 64-byte LDS row segment
 constexpr int GNS = 4;               // LDS ring stages
 constexpr int WAVES_N = 4;                   // waves along n; 2 along m
 constexpr int WAVES_M = 2;
-constexpr int NBW = GBN / 16 / WAVES_N;      // 16-row W blocks per wave
+static_assert(NBW == GBN / 16 / WAVES_N, "64 n per wave");
 constexpr int GTHR = 64 * WAVES_N * WAVES_M;
 constexpr int GROUP_M = 4;           // row tiles per raster group
-constexpr int W_REG_H = GBN * GBK;   // halves in the W region of a stage (16 KB)
 constexpr int W_DMA = W_REG_H * 2 / (GTHR * 16);  // 16-byte W pieces per thread per k tile
 
 // MB: 16-row activation blocks per wave; the workgroup's activation tile is 32*MB rows
@@ -56,205 +50,6 @@ struct Tile {
 constexpr int A_DMA = Tile<8>::A_REG_H * 2 / (GTHR * 16);
 constexpr int DMA_PER_TILE = W_DMA + A_DMA;
 static_assert(Tile<8>::A_REG_H * 2 == A_DMA * GTHR * 16 && Tile<7>::A_REG_H * 2 > (A_DMA - 1) * GTHR * 16, "A pieces");
-
-typedef __attribute__((address_space(3))) half8 lds_half8;
-typedef float f2v __attribute__((ext_vector_type(2)));
-
-// s_waitcnt vmcnt(N) (lgkmcnt and expcnt left alone). A device function, so that the host pass never checks
-// the builtin's constant argument inside the kernel template (where it depends on the tile height).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | ((N >> 4) << 14));
-}
-
-struct GemmParams {
-    const _Float16* a;
-    const _Float16* w;
-    const _Float16* a2;
-    const _Float16* w2;
-    int K, K2, M, N;
-    void* c;
-    int ldc;
-    const float* gate;
-    float beta;
-    int tiles_m, tiles_n, total, per;
-    int pairs;  // output rows or base not 16-byte (fp32) / 8-byte (fp16) aligned: store element pairs
-    int wprep;  // w is in the prepared tile layout (kiln_linear16_prepare_weight), not [N, K] rows
-    // EPI_QKV (the DiT self-attention projection with its QK-RMSNorm, RoPE and fp16 K/V preparation fused):
-    // columns [0, D) are Q, [D, 2D) K, [2D, 3D) V of H heads; row r is token r % T of item r / T
-    _Float16* q16;      // [M, D]: fp16(rope(rmsnorm(q)) * qscale)
-    uint16_t* kvp[MAX_JOBS];  // prepared K/V per item (common.hpp layout), K = rope(rmsnorm(k))
-    int T, H;
-    const uint16_t* qw;  // bf16 [128] norm weights
-    const uint16_t* kw;
-    float eps, qscale;
-    const float* rcos;  // [T, 64]
-    const float* rsin;
-};
-constexpr int EPI_QKV = 4;
-struct KvTailJobs {
-    uint16_t* kvp[MAX_JOBS];
-};
-
-__device__ __forceinline__ floatx4 mfma16(half8 a, half8 b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
-// GELU(v) = v Phi(v) = v (1 + erf(v / sqrt 2)) / 2, with Phi from erfc, which keeps its relative accuracy in the
-// negative tail: Phi(v) = erfc(z) / 2 for v < 0 and 1 - erfc(z) / 2 for v >= 0, z = |v| / sqrt 2. erfc(z) for
-// z >= 0 is the Chebyshev approximation "erfcc" of Numerical Recipes in C (Press et al., 2nd ed., section 6.2),
-// fractional error below 1.2e-7 everywhere: ~17 VALU operations and no branches, about half of a library erff,
-// and far below the fp16 output's rounding.
-__device__ __forceinline__ float gelu_erf(float v) {
-    const float z = fabsf(v) * 0.70710678118654752f;
-    const float t = __builtin_amdgcn_rcpf(1.f + 0.5f * z);
-    float r = 0.17087277f;
-    r = fmaf(t, r, -0.82215223f);
-    r = fmaf(t, r, 1.48851587f);
-    r = fmaf(t, r, -1.13520398f);
-    r = fmaf(t, r, 0.27886807f);
-    r = fmaf(t, r, -0.18628806f);
-    r = fmaf(t, r, 0.09678418f);
-    r = fmaf(t, r, 0.37409196f);
-    r = fmaf(t, r, 1.00002368f);
-    r = fmaf(t, r, -1.26551223f);
-    const float half_erfc = 0.5f * t * __expf(r - z * z);
-    return v * (v >= 0.f ? 1.f - half_erfc : half_erfc);
-}
-
-// EPI_QKV epilogue. The workgroup's 256 columns are two heads of one region (Q, K or V: D is a multiple of 256).
-// A wave holds 64 columns = half a head; its partner wave (wv ^ 2, the same rows) holds the other half. In the Q and
-// K regions the k loop read the wave's W blocks so that block nb holds head dims dq(nb) + 0..15, dq(nb) =
-// 32*(wn & 1) + 16*(nb & 1) + 64*(nb >> 1): each RoPE pair (i, i + 64) is element (nb, e) and (nb + 2, e) of one
-// lane. Q/K: per-row sum of squares over the head (own half + partner's, through LDS), scale by rsqrt(mean + eps)
-// and the bf16 weight, then RoPE in registers. Q is stored as fp16(q * qscale) rows, K and V in the prepared K/V
-// layout of their item (kv_k_el / kv_v_el).
-template <int MB>
-__device__ __forceinline__ void qkv_epilogue(const GemmParams& p, floatx4 (&acc)[NBW][MB], _Float16* lds, int m0,
-                                             int n0, int wv, int wn, int wm, int lane) {
-    const int D = p.H * HD;
-    const int region = n0 / D, c0 = n0 - region * D;
-    const int hd = (c0 + (wn >> 1) * HD) / HD, half = wn & 1;
-    const int rl = lane & 15, cq = 4 * (lane >> 4);  // column within a 16-column block: cq + e
-    const int rbase = m0 + wm * 16 * MB + rl;
-    auto dq = [&](int nb) { return 32 * half + 16 * (nb & 1) + 64 * (nb >> 1); };  // Q/K head dim of block nb
-    float* lf = reinterpret_cast<float*>(lds);
-    __syncthreads();  // every wave is done with the k loop's LDS stages
-    if (region < 2) {
-        const uint16_t* w = region == 0 ? p.qw : p.kw;
-        float wt[NBW][4];
-#pragma unroll
-        for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) wt[nb][e] = bf16_to_f32(w[dq(nb) + cq + e]);  // any alignment of w
-        float r[MB];
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) {
-            float ss = 0.f;
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) ss += acc[nb][mb][e] * acc[nb][mb][e];
-            ss += __shfl_xor(ss, 16, 64);
-            ss += __shfl_xor(ss, 32, 64);
-            if (lane < 16) lf[wv * 16 * MB + mb * 16 + rl] = ss;
-            r[mb] = ss;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) r[mb] = rsqrtf((r[mb] + lf[(wv ^ 2) * 16 * MB + mb * 16 + rl]) * (1.0f / HD) + p.eps);
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) acc[nb][mb][e] *= r[mb] * wt[nb][e];
-        if (p.rcos) {  // RoPE (none for the cross-attention Q projection)
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) {
-                const int row = rbase + mb * 16;
-                const int t = (row < p.M ? row : 0) % p.T;
-#pragma unroll
-                for (int nb = 0; nb < 2; nb++) {
-                    const floatx4 cs = *reinterpret_cast<const floatx4*>(p.rcos + (size_t)t * 64 + dq(nb) + cq);
-                    const floatx4 sn = *reinterpret_cast<const floatx4*>(p.rsin + (size_t)t * 64 + dq(nb) + cq);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        const float a = acc[nb][mb][e], b = acc[nb + 2][mb][e];
-                        acc[nb][mb][e] = a * cs[e] - b * sn[e];
-                        acc[nb + 2][mb][e] = b * cs[e] + a * sn[e];
-                    }
-                }
-            }
-        }
-    }
-    if (region == 2 && p.T % 32 == 0) {
-        // V through LDS, one head (128 columns) per pass: the wave pairs of that head write their fp16 values
-        // row-major (rows padded to 288 bytes), then every wave assembles whole 16-byte V^T operand units (8 keys of
-        // one d) with transposing reads, as the K/V prepare pass does, instead of 2-byte scatters. With T a
-        // multiple of 32 (and the tile's first row one too) no 32-key half tile straddles two items.
-        constexpr int VRS = HD + 16, BM = 32 * MB;
-        static_assert(BM * VRS <= GNS * Tile<MB>::STAGE_H, "the staged V tile fits in the ring's LDS");
-        const int i = lane & 15, gq = lane >> 4;
-        typedef short s4 __attribute__((ext_vector_type(4)));
-        typedef short s8 __attribute__((ext_vector_type(8)));
-        typedef __attribute__((address_space(3))) s4 lds_s4;
-#pragma unroll
-        for (int pass = 0; pass < 2; pass++) {
-            if ((wn >> 1) == pass) {
-#pragma unroll
-                for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-                    for (int nb = 0; nb < NBW; nb++) {
-                        const floatx4 v = acc[nb][mb];
-                        *reinterpret_cast<half4*>(lds + (wm * 16 * MB + mb * 16 + rl) * VRS + half * 64 + nb * 16 + cq) =
-                            half4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-                    }
-            }
-            __syncthreads();
-            const int hdp = (c0 + pass * HD) / HD;
-            for (int op = wv; op < (BM / 32) * 8; op += WAVES_N * WAVES_M) {
-                const int ht = op >> 3, db = op & 7, row0 = m0 + ht * 32;
-                if (row0 >= p.M) break;  // ops ascend with ht: every later one is past the matrix too
-                const int b = row0 / p.T, key0 = row0 - b * p.T;
-                const _Float16* src = lds + (ht * 32 + 4 * gq + (i >> 2)) * VRS + 16 * db + 4 * (i & 3);
-                const s4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)src);
-                const s4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)(src + 16 * VRS));
-                _Float16* kv = reinterpret_cast<_Float16*>(p.kvp[b]) + (size_t)hdp * kv_head_stride(p.T) +
-                               (size_t)(key0 / KT) * KV_TILE_H;
-                *reinterpret_cast<s8*>(kv + kv_v_off((key0 % KT) / 32, db, lane)) =
-                    s8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            }
-            __syncthreads();  // every read of this head's values precedes the next pass's writes
-        }
-        return;
-    }
-#pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-        const int row = rbase + mb * 16;
-        if (row >= p.M) continue;
-        const int b = row / p.T, key = row - b * p.T;
-        _Float16* kv = reinterpret_cast<_Float16*>(p.kvp[b]) + (size_t)hd * kv_head_stride(p.T) +
-                       (size_t)(key / KT) * KV_TILE_H;
-        const int kc = (key % KT) / 32, k32 = key % 32;
-#pragma unroll
-        for (int nb = 0; nb < NBW; nb++) {
-            // 4 consecutive d, inside one 8-element chunk (Q/K: the permuted head dims; V: the plain ones)
-            const int d = (region < 2 ? dq(nb) : half * 64 + nb * 16) + cq;
-            const floatx4 v = acc[nb][mb];
-            if (region == 0) {
-                *reinterpret_cast<half4*>(p.q16 + (size_t)row * D + hd * HD + d) =
-                    half4{(_Float16)(v[0] * p.qscale), (_Float16)(v[1] * p.qscale), (_Float16)(v[2] * p.qscale),
-                          (_Float16)(v[3] * p.qscale)};
-            } else if (region == 1) {
-                *reinterpret_cast<half4*>(kv + kv_k_el(kc, k32, d)) =
-                    half4{(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++) kv[kv_v_el(kc, k32, d + e)] = (_Float16)v[e];
-            }
-        }
-    }
-}
 
 // LATE (prepared weights): in steady steps the refill DMA leaves the barrier's shadow and the two waves of a SIMD
 // issue it at different points of the MFMA stream: waves 0-3 after the first activation block's MFMAs, waves 4-7
@@ -304,9 +99,6 @@ __global__ __launch_bounds__(GTHR, 1) void k_gemm16(const GemmParams p) {
         }
     };
     voffs(p.K, p.wprep != 0, voff_w, voff_a);
-#define GEMM_RSRC(base, bytes)                                                                             \
-    __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(base), (short)0, (int)min((size_t)(bytes), (size_t)0x7fffffff), \
-                                      0x00020000 /* raw, CDNA */)
     const __amdgpu_buffer_rsrc_t rw1 =
         p.wprep ? GEMM_RSRC(p.w + (size_t)tn * GBN * p.K, (size_t)GBN * p.K * 2)
                 : GEMM_RSRC(p.w + (size_t)n0 * p.K, (size_t)nrows * p.K * 2);
@@ -449,7 +241,7 @@ __global__ __launch_bounds__(GTHR, 1) void k_gemm16(const GemmParams p) {
     if (kt < KTT) step(False{}, kt, fw, gw);
 
     if constexpr (EPI == EPI_QKV) {
-        qkv_epilogue<MB>(p, acc, lds, m0, n0, wv, wn, wm, lane);
+        qkv_epilogue<WAVES_N, WAVES_M, MB, 1, GNS * STAGE_H>(p, acc, lds, m0, n0, wv, wn, wm, 0, lane);
         return;
     }
     // epilogue: lane holds rows m0 + wm*16*MB + mb*16 + (lane & 15), columns n0 + wn*64 + nb*16 + 4*(lane >> 4) + e
@@ -457,67 +249,14 @@ __global__ __launch_bounds__(GTHR, 1) void k_gemm16(const GemmParams p) {
     const int ncol = n0 + wn * NBW * 16 + 4 * (lane >> 4);
     if (ncol >= p.N) return;  // a column range of the last tile past N (N % 256 == 128)
     floatx4 gv[NBW];
-    if constexpr (EPI == KILN_EPI_RESID) {
 #pragma unroll
-        for (int nb = 0; nb < NBW; nb++) {
-            if (p.gate) {
-                const float* g = p.gate + ncol + nb * 16;
-                gv[nb] = floatx4{g[0], g[1], g[2], g[3]};
-            } else {
-                gv[nb] = floatx4{1.f, 1.f, 1.f, 1.f};
-            }
-        }
-    }
+    for (int nb = 0; nb < NBW; nb++) gv[nb] = gate_of<EPI>(p, ncol + nb * 16);
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
         const int m = mrow + mb * 16;
         if (m >= p.M) break;
 #pragma unroll
-        for (int nb = 0; nb < NBW; nb++) {
-            const int n = ncol + nb * 16;
-            const size_t off = (size_t)m * p.ldc + n;
-            const floatx4 v = acc[nb][mb];
-            if constexpr (EPI == KILN_EPI_F32 || EPI == KILN_EPI_RESID) {
-                float* dst = static_cast<float*>(p.c) + off;
-                floatx4 o;
-                const bool need_old = EPI == KILN_EPI_RESID || p.beta != 0.f;
-                if (need_old) {
-                    if (!p.pairs) {
-                        o = *reinterpret_cast<const floatx4*>(dst);
-                    } else {
-                        const f2v o0 = reinterpret_cast<const f2v*>(dst)[0], o1 = reinterpret_cast<const f2v*>(dst)[1];
-                        o = floatx4{o0[0], o0[1], o1[0], o1[1]};
-                    }
-                }
-                floatx4 r;
-                if constexpr (EPI == KILN_EPI_RESID) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) r[e] = o[e] + gv[nb][e] * v[e];
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) r[e] = need_old ? v[e] + p.beta * o[e] : v[e];
-                }
-                if (!p.pairs) {
-                    *reinterpret_cast<floatx4*>(dst) = r;
-                } else {
-                    reinterpret_cast<f2v*>(dst)[0] = f2v{r[0], r[1]};
-                    reinterpret_cast<f2v*>(dst)[1] = f2v{r[2], r[3]};
-                }
-            } else {
-                _Float16* dst = static_cast<_Float16*>(p.c) + off;
-                floatx4 r = v;
-                if constexpr (EPI == KILN_EPI_GELU16) {
-#pragma unroll
-                    for (int e = 0; e < 4; e++) r[e] = gelu_erf(v[e]);
-                }
-                if (!p.pairs) {
-                    *reinterpret_cast<half4*>(dst) = half4{(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
-                } else {
-                    reinterpret_cast<half2v*>(dst)[0] = half2v{(_Float16)r[0], (_Float16)r[1]};
-                    reinterpret_cast<half2v*>(dst)[1] = half2v{(_Float16)r[2], (_Float16)r[3]};
-                }
-            }
-        }
+        for (int nb = 0; nb < NBW; nb++) store_out<EPI>(p, m, ncol + nb * 16, acc[nb][mb], gv[nb]);
     }
 }
 
@@ -562,6 +301,9 @@ hipError_t launch_gemm_wprep(uint16_t* wp, const uint16_t* w, int N, int K, bool
     return hipGetLastError();
 }
 
+struct KvTailJobs {
+    uint16_t* kvp[MAX_JOBS];
+};
 __global__ void k_kv_zero_tail(KvTailJobs j, size_t head_stride, size_t tail_off) {
     // block (item, head): 32 KB of the last tile, 16 bytes per thread and step
     _Float16* base = reinterpret_cast<_Float16*>(j.kvp[blockIdx.y]) + blockIdx.x * head_stride + tail_off;
@@ -617,16 +359,17 @@ static hipError_t launch_mb(GemmParams p, int epi, hipStream_t s) {
 // Activation tile height (32*MB rows, MB in {8, 7}): the one with the fewest CU rounds x rows per tile, one
 // workgroup per CU. M = 6912 (the DiT's CFG batch) is 27 tiles of 256 rows, so every grid of 256-row tiles
 // leaves 5/32 of the last round idle; 224-row tiles give 31 per column and fill 97%.
-int gemm16_mb(int M, int N) {
-    const int cus = cu_count(), tn = (N + GBN - 1) / GBN;
+static int gemm16_mb(int M, int N, int cus, long* tiles) {
+    const int tn = (N + GBN - 1) / GBN;
     int best = 8;
     long best_cost = -1;
     for (int mb : {8, 7}) {
-        const long tiles = (long)((M + 32 * mb - 1) / (32 * mb)) * tn;
-        const long cost = (tiles + cus - 1) / cus * mb;
+        const long t = (long)((M + 32 * mb - 1) / (32 * mb)) * tn;
+        const long cost = (t + cus - 1) / cus * mb;
         if (best_cost < 0 || cost < best_cost) {
             best = mb;
             best_cost = cost;
+            *tiles = t;
         }
     }
     return best;
@@ -661,7 +404,16 @@ hipError_t launch_gemm16(const GemmLaunch& g, hipStream_t s) {
         p.rcos = g.rcos;
         p.rsin = g.rsin;
     }
-    if (gemm16_mb(g.M, g.N) == 7) return launch_mb<7>(p, g.epi, s);
+    // Few rows leave most CUs without a 256-wide tile: M = 256 x 2048 x 2048 takes 42.9 us on this kernel's 16 tiles
+    // and 9.1 us on 64 x 32 ones, M = 1024 45.0 against 17.5 (128 x 64), M = 3072 47.8 against 35.2 (128 x 192); at
+    // M = 6912 it is 62.5 against 93.8. The models meet near the size where the large tiles fill the chip.
+    const int cus = cu_count();
+    long tiles = 0;
+    const int mb = gemm16_mb(g.M, g.N, cus, &tiles);
+    const SmallGemm small = gemm16s_choose(g.M, g.N, g.K + g.K2, g.epi, cus);
+    const double large = gemm_cost({0.66, 1.17 * mb, 0.0663 * mb, 0.0396 * mb}, tiles, (g.K + g.K2) / GBK, cus);
+    if (small.cost < large) return launch_gemm16s(p, small.cfg, g.epi, s);
+    if (mb == 7) return launch_mb<7>(p, g.epi, s);
     return launch_mb<8>(p, g.epi, s);
 }
 
