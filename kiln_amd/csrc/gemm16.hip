@@ -319,7 +319,7 @@ hipError_t launch_kv_zero_tail(uint16_t* const* kvp, int njobs, int T, int H, hi
     return hipGetLastError();
 }
 
-static int cu_count() {
+int cu_count() {
     static int cus[64] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;

@@ -1,0 +1,70 @@
+"""GPU parity of the fp32 linear layers with bf16 weights (kiln_linear_f32) on the bf16 matrix cores, where an fp32
+input is split into three bf16 parts without a remainder: every tile, its edges, and values at the ends of fp32.
+
+Bar: fp32 sums of exact products, |err| <= sqrt(cols) 2^-21 sum_k |x_k w_k| (the bar of the fp16 GEMM's fp32 sums).
+"""
+import numpy as np
+import pytest
+import torch
+
+import kiln_amd
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _check(y, x, w, what=""):
+    ref = x.double() @ w.double().T
+    bar = w.shape[1] ** 0.5 * 2.0 ** -21 * (x.double().abs() @ w.double().abs().T) + 1e-44
+    err = (y.double() - ref).abs()
+    assert torch.isfinite(y).all(), what
+    assert (err <= bar).all(), f"{what}: {(err / bar).max().item():.2f} of the bar"
+
+
+# the five tiles (256 x 128, 128 x 128, 128 x 64, 128 x 32, 64 x 32), a row over and under an edge, rows that end
+# inside a tile and inside a group of four columns, a partial last step of 2, 4 or 8 slices
+@pytest.mark.parametrize("T,rows,cols", [(4097, 2048, 96), (2047, 2048, 352), (1025, 2048, 160), (500, 2050, 288), (65, 129, 64),
+                                         (33, 64, 2080), (1, 3, 32), (6912, 64, 256), (31, 2048, 1056)])
+def test_linear_f32_tiles(gpu, T, rows, cols):
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn(T, cols, device=DEV, generator=g)
+    w = (torch.randn(rows, cols, device=DEV, generator=g) * cols ** -0.5).bfloat16()
+    buf = torch.full((T + 2, rows + 1), float("nan"), device=DEV)  # an odd row stride: element stores
+    for y in (torch.full((T, rows), float("nan"), device=DEV), buf[1:T + 1, :rows]):
+        kiln_amd.linear_f32(y, x, w)
+        _check(y, x, w)
+    assert torch.isnan(buf[0]).all() and torch.isnan(buf[T + 1]).all() and torch.isnan(buf[:, rows]).all()
+    wide = torch.randn(T, cols + 4, device=DEV, generator=g)[:, :cols]  # a row stride of its own
+    kiln_amd.linear_f32(buf[1:T + 1, :rows], wide, w)
+    _check(buf[1:T + 1, :rows], wide, w)
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -20, 2.0 ** 100])
+def test_linear_f32_scales(gpu, scale):
+    """Far from 1 the three parts keep all 24 bits."""
+    g = torch.Generator(device=DEV).manual_seed(1)
+    x = torch.randn(70, 256, device=DEV, generator=g) * scale
+    w = torch.randn(130, 256, device=DEV, generator=g).bfloat16()
+    y = torch.empty(70, 130, device=DEV)
+    kiln_amd.linear_f32(y, x, w)
+    _check(y, x, w)
+
+
+def test_linear_f32_infinities_and_nan(gpu):
+    """The same non-finite outputs as the general form (x one float off its alignment takes it)."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    buf = torch.randn(96 * 64 + 1, device=DEV, generator=g)
+    x = buf[1:].view(96, 64)
+    w = torch.randn(128, 64, device=DEV, generator=g).bfloat16()
+    x[3, 5], x[7, 0], x[9, 63], x[11, 1] = float("inf"), float("-inf"), float("nan"), 0.0
+    x[20] = 1.0  # no remainders
+    w[4, 7], w[6, 1], w[8, 2], w[8, 3] = float("inf"), float("-inf"), float("nan"), 0.0
+    x[30, 9] = 3.4e38
+    ya, yb = torch.empty(96, 128, device=DEV), torch.empty(96, 128, device=DEV)
+    kiln_amd.linear_f32(ya, x, w)
+    kiln_amd.linear_f32(yb, x.clone(), w)
+    a, b = ya.cpu().numpy(), yb.cpu().numpy()
+    assert (np.isnan(a) == np.isnan(b)).all()
+    assert (np.isposinf(a) == np.isposinf(b)).all() and (np.isneginf(a) == np.isneginf(b)).all()
+    f = np.isfinite(a)
+    assert np.abs(a[f] - b[f]).max() <= 1e-5 * np.abs(a[f]).max()
