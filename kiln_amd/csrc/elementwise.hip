@@ -78,17 +78,17 @@ __device__ __forceinline__ float ldv(const _Float16* p) { return (float)*p; }
 __device__ __forceinline__ void stv(float* p, float v) { *p = v; }
 __device__ __forceinline__ void stv(_Float16* p, float v) { *p = (_Float16)v; }
 
-// ---- modulated LayerNorm of the DiT block (engine/src/kernels.cu:678-697): one wave per row ----
+// ---- modulated LayerNorm of the DiT block (engine/src/kernels.cu:678-697) ----
 // y = (x - mean) * rsqrt(var + eps) * (1 + scale) + shift, mean and var over the row (two passes, as the
-// reference). Rows of up to 64 lanes x NC float4 chunks stay in registers: one HBM read, one write.
+// reference). A row stays in the registers of a wave (rows of up to 512) or a workgroup: one HBM read, one write.
 __device__ __forceinline__ void st4(float* p, floatx4 v) { *reinterpret_cast<floatx4*>(p) = v; }
 __device__ __forceinline__ void st4(_Float16* p, floatx4 v) {
     half4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
     *reinterpret_cast<half4*>(p) = h;
 }
 
-// A wave normalizes LN_RPW consecutive rows with the modulation vectors loaded once (per row they would be twice
-// the row's own bytes in L2 reads; 6912 x 2048 fp16 out: 15.4 -> 14.4 us against one row per wave).
+// Short rows: a wave normalizes LN_RPW consecutive ones with the modulation vectors loaded once (per row they would
+// be twice the row's own bytes in L2 reads).
 constexpr int LN_RPW = 4;
 template <typename OutT, int NC>
 __global__ __launch_bounds__(256) void k_layernorm_mod_rows(OutT* y, const float* x, const float* scale,
@@ -140,6 +140,51 @@ __global__ __launch_bounds__(256) void k_layernorm_mod_rows(OutT* y, const float
     }
 }
 
+// Rows of the DiT's width: a row to a workgroup, at most NC float4 chunks to a thread. HBM-bound with many rows,
+// where it equals the form above (6912 x 2048, fp16 out, rows from memory: 19.1 against 19.5 us); with few rows that
+// form's wave walks 4 rows in turn on a handful of CUs: 256 x 2048 5.2 -> 2.4 us, 1024 6.3 -> 4.1, 3072 8.6 -> 7.6.
+template <typename OutT, int NC>
+__global__ __launch_bounds__(256) void k_layernorm_mod_wg(OutT* y, const float* x, const float* scale, const float* shift,
+                                                          int rows, int dim, float eps) {
+    __shared__ float red[4];
+    const int row = blockIdx.x, nc = dim / 4, t = threadIdx.x;
+    const float* xr = x + (size_t)row * dim;
+    OutT* yr = y + (size_t)row * dim;
+    floatx4 v[NC], sc[NC], sh[NC];
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const int c = min(t + 256 * k, nc - 1);
+        v[k] = *reinterpret_cast<const floatx4*>(xr + 4 * c);
+        sc[k] = *reinterpret_cast<const floatx4*>(scale + 4 * c);
+        sh[k] = *reinterpret_cast<const floatx4*>(shift + 4 * c);
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+        if (t + 256 * k < nc) s += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+    const float mean = block_sum256(s, red) / (float)dim;
+    float q = 0.f;
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+        if (t + 256 * k < nc)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float d = v[k][e] - mean;
+                q += d * d;
+            }
+    const float r = rsqrtf(block_sum256(q, red) / (float)dim + eps);
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const int c = t + 256 * k;
+        if (c < nc) {
+            floatx4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++) o[e] = (v[k][e] - mean) * r * (1.f + sc[k][e]) + sh[k][e];
+            st4(yr + 4 * c, o);
+        }
+    }
+}
+
 // any dim / alignment: three passes over the row (the second and third hit the cache)
 template <typename OutT>
 __global__ __launch_bounds__(256) void k_layernorm_mod_any(OutT* y, const float* x, const float* scale,
@@ -166,9 +211,9 @@ static hipError_t layernorm_mod_sel(OutT* y, const float* x, const float* scale,
     const dim3 grid((rows + 3) / 4), block(256), grid_rows((rows + 4 * LN_RPW - 1) / (4 * LN_RPW));
     const int nc = dim / 4;
     if (vec && nc <= 64 * 2) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 2>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
-    else if (vec && nc <= 64 * 4) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 4>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
-    else if (vec && nc <= 64 * 8) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 8>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
-    else if (vec && nc <= 64 * 16) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 16>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
+    else if (vec && nc <= 256) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 1>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);
+    else if (vec && nc <= 256 * 2) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 2>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);
+    else if (vec && nc <= 256 * 4) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 4>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);
     else hipLaunchKernelGGL((k_layernorm_mod_any<OutT>), grid, block, 0, s, y, x, scale, shift, rows, dim, eps);
     return hipGetLastError();
 }

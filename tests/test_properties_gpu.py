@@ -166,3 +166,18 @@ def test_identical_keys_give_mean_value(gpu, Tk):
     err = (o.double() - mean).abs().max().item()
     print(f"[parity] identical keys: max |out - mean(V)| = {err:.3e}", flush=True)
     assert err <= 2e-4  # |mean| ~ 0.02-0.1: fp16 rounding of the output (<= 2^-14) and fp32 sums of Tk terms
+
+
+@pytest.mark.parametrize("rows,dim", [(1, 512), (3, 516), (2, 1024), (5, 1028), (257, 2048), (2, 2052), (3, 4096), (2, 4100)])
+def test_layernorm_mod_row_forms(gpu, rows, dim):
+    """The widths on both sides of each row form's edge against a float64 LayerNorm: fp32 rounding of the row's sums
+    and of the modulation (a few ulp of the largest term)."""
+    g = torch.Generator().manual_seed(dim)
+    x, sc, sh = torch.randn(rows, dim, generator=g) * 3 + 1, torch.randn(dim, generator=g), torch.randn(dim, generator=g)
+    ref = torch.nn.functional.layer_norm(x.double(), (dim,), eps=1e-6) * (1 + sc.double()) + sh.double()
+    y = torch.full((rows, dim), float("nan"), device=DEV)
+    kiln_amd.layernorm_mod(y, x.to(DEV), sc.to(DEV), sh.to(DEV))
+    assert (y.cpu().double() - ref).abs().max() <= 2.0 ** -20 * ref.abs().max()
+    y16 = torch.full((rows, dim), float("nan"), device=DEV, dtype=torch.float16)
+    kiln_amd.layernorm_mod(y16, x.to(DEV), sc.to(DEV), sh.to(DEV))
+    assert (y16.cpu().double() - ref).abs().max() <= 2.0 ** -11 * ref.abs().max() + 2.0 ** -20 * ref.abs().max()
