@@ -274,6 +274,11 @@ int kiln_kv_prepare(uint16_t* kvp, const void* k, int ldk, const void* v, int ld
                     const uint16_t* k_norm_w, float eps, const float* rope_cos, const float* rope_sin,
                     kiln_stream_t stream);
 
+/* The same for `blocks` layers at once: kv [Tk, ld] fp32 rows hold block b's K at column b*2*H*128 and its V H*128
+ * columns further; k_norm_w bf16 [blocks, 128]. kvp: blocks x kiln_kv_prepped_bytes(Tk, H), one after the other. */
+int kiln_kv_prepare_blocks(uint16_t* kvp, const float* kv, int ld, int blocks, int Tk, int H, const uint16_t* k_norm_w,
+                           float eps, kiln_stream_t stream);
+
 /* Attention of Q [Tq, ldq] (in_dtype) against a prepared K/V buffer. The Q tile load applies the
  * optional per-head RMSNorm (q_norm_w, eps) and RoPE (tables [Tq, 64]) before the fp16 rounding. */
 int kiln_attn_fwd_prepped(void* out, int out_dtype, int ldo, const void* q, int in_dtype, int ldq,

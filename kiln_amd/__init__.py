@@ -77,6 +77,7 @@ _SIGS = {
     "kiln_cosmos_rope_tables": (_i, [_vp, _vp, _i, _i]),
     "kiln_kv_prepped_bytes": (_sz, [_i, _i]),
     "kiln_kv_prepare": (_i, [_vp, _vp, _i, _vp, _i, _i, _i, _i, _vp, _f, _vp, _vp, _vp]),
+    "kiln_kv_prepare_blocks": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _f, _vp]),
     "kiln_attn_fwd_prepped": (_i, [_vp, _i, _i, _vp, _i, _i, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "kiln_attn_fwd_prepped_batch": (_i, [_vp, _i, _i, _ll, _vp, _i, _i, _ll, _vp, _f, _vp, _vp, _vp, _i, _i, _i, _i,
                                          _i, _vp]),

@@ -643,7 +643,8 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 struct PrepParams {
     KVPrepJob job[MAX_JOBS];  // blockIdx.z selects the job
     int Tk, tpb;              // keys; 32-key half tiles per block
-    const uint16_t* kw;
+    int hpg, gcols;           // heads of a group, and the columns between its last head and the next group's first
+    const uint16_t* kw;       // [128] of every group
     float eps;
     const float* rcos;
     const float* rsin;
@@ -663,7 +664,8 @@ __global__ __launch_bounds__(256) void k_kv_prep(const PrepParams p) {
     // V half tile in fp16, rows padded to 288 bytes: the transposing reads of one 16-lane group touch 4 rows
     // 8 banks apart, conflict-free
     __shared__ __attribute__((aligned(16))) _Float16 vt[32][HD + 16];
-    const int tid = threadIdx.x, h = blockIdx.y;
+    const int tid = threadIdx.x, h = blockIdx.y, grp = h / p.hpg;
+    const int col = h * HD + grp * p.gcols;
     const KVPrepJob& jb = p.job[blockIdx.z];
     const int Tk = p.Tk, nhalf = 2 * kv_tiles(Tk);
     const int t0 = blockIdx.x * p.tpb, t1 = min(t0 + p.tpb, nhalf);
@@ -676,13 +678,13 @@ __global__ __launch_bounds__(256) void k_kv_prep(const PrepParams p) {
 #pragma unroll
     for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int e = 0; e < 8; e++) kwf[c][e] = KNORM ? bf16_to_f32(p.kw[8 * (q8 + 8 * c) + e]) : 1.f;
+        for (int e = 0; e < 8; e++) kwf[c][e] = KNORM ? bf16_to_f32(p.kw[grp * HD + 8 * (q8 + 8 * c) + e]) : 1.f;
 
     auto load_half = [&](int jh, PrepHalf<InT, ROPE>& t) {
         const int key = jh * 32 + kk;
         if (key < Tk) {
-            const InT* kr = k + (size_t)key * jb.ldk + h * HD + 8 * q8;
-            const InT* vr = v + (size_t)key * jb.ldv + h * HD + 16 * q8;
+            const InT* kr = k + (size_t)key * jb.ldk + col + 8 * q8;
+            const InT* vr = v + (size_t)key * jb.ldv + col + 16 * q8;
             t.k[0].load(kr);
             t.k[1].load(kr + 64);
             t.v[0].load(vr);
@@ -947,7 +949,7 @@ static hipError_t dispatch_prep(const PrepParams& p, int njobs, int H, hipStream
 }
 
 hipError_t launch_kv_prep(const KVPrepJob* jobs, int njobs, DT in, int Tk, int H, const uint16_t* kw, float eps,
-                          const float* rcos, const float* rsin, hipStream_t s) {
+                          const float* rcos, const float* rsin, hipStream_t s, int hpg, int gcols) {
     if (Tk <= 0 || H <= 0 || njobs <= 0) return hipSuccess;
     if (njobs > MAX_JOBS) return hipErrorInvalidValue;
     PrepParams p{};
@@ -957,6 +959,8 @@ hipError_t launch_kv_prep(const KVPrepJob* jobs, int njobs, DT in, int Tk, int H
     // the first is converted and stored (measured best at T = 1536 and 4096; one per block for small inputs)
     const int halves = 2 * kv_tiles(Tk) * H * njobs;
     p.tpb = halves >= 1024 ? 2 : 1;
+    p.hpg = hpg > 0 ? hpg : H;
+    p.gcols = gcols;
     p.kw = kw;
     p.eps = eps;
     p.rcos = rcos;

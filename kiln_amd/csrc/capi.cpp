@@ -284,6 +284,21 @@ int kiln_kv_prepare(uint16_t* kvp, const void* k, int ldk, const void* v, int ld
                      "kv_prep launch");
 }
 
+int kiln_kv_prepare_blocks(uint16_t* kvp, const float* kv, int ld, int blocks, int Tk, int H, const uint16_t* k_norm_w,
+                           float eps, kiln_stream_t stream) {
+    kiln::prof::Scope prof_("attention", (hipStream_t)stream);
+    if (Tk < 0 || H <= 0 || blocks <= 0 || blocks > 65535 / H || ld < blocks * 2 * H * kiln::HD)
+        return fail(KILN_EINVAL, "bad sizes Tk=%d H=%d blocks=%d ld=%d", Tk, H, blocks, ld);
+    if (Tk > MAX_TK) return fail(KILN_EUNSUPPORTED, "Tk=%d above %d keys per head", Tk, MAX_TK);
+    if (Tk == 0) return KILN_OK;
+    if (!kvp || !kv || !k_norm_w) return fail(KILN_EINVAL, "null pointer");
+    if (!aligned16(kvp) || !rows_ok(kv, ld, DT::F32)) return fail(KILN_EUNSUPPORTED, "kvp / K/V rows not 16-byte aligned");
+    const kiln::KVPrepJob pj{kvp, kv, kv + H * kiln::HD, ld, ld};
+    return hip_check(kiln::launch_kv_prep(&pj, 1, DT::F32, Tk, H * blocks, k_norm_w, eps, nullptr, nullptr,
+                                          (hipStream_t)stream, H, H * kiln::HD),
+                     "kv_prep launch");
+}
+
 int kiln_attn_fwd_prepped(void* out, int out_dtype, int ldo, const void* q, int in_dtype, int ldq,
                           const uint16_t* q_norm_w, float eps, const float* rope_cos, const float* rope_sin,
                           const uint16_t* kvp, int Tq, int Tk, int H, int npad, kiln_stream_t stream) {

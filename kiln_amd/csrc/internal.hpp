@@ -52,9 +52,10 @@ struct KVPrepJob {
     const void* v;
     int ldk, ldv;
 };
-// Prepares njobs (<= MAX_JOBS) contexts of Tk keys and H heads in one launch (K RMSNorm with kw, RoPE).
+// Prepares njobs (<= MAX_JOBS) contexts of Tk keys and H heads in one launch (K RMSNorm with kw, RoPE). hpg > 0: the
+// heads come in groups of hpg, a group's first head gcols columns after the last one's end, with kw [128] of its own.
 hipError_t launch_kv_prep(const KVPrepJob* jobs, int njobs, DT in, int Tk, int H, const uint16_t* kw, float eps,
-                          const float* rcos, const float* rsin, hipStream_t s);
+                          const float* rcos, const float* rsin, hipStream_t s, int hpg = 0, int gcols = 0);
 
 // acc = a [M,K] w[N,K]^T (+ a2 [M,K2] w2[N,K2]^T), all fp16 dense rows; epilogue `epi` (kiln_epi) into c (row
 // stride ldc). N % 128 == 0, K % 32 == 0, K2 % 32 == 0, 16-byte aligned operand bases.

@@ -80,9 +80,9 @@ static DeviceBuffer prep16(const uint16_t* src_bf16, int rows, int cols, hipStre
 struct Dit::Block {
     // fp16 path: prepared fp16 weights
     DeviceBuffer qkv16, sa_o16, ca_q16, ca_o16, mlp1_16, mlp2_16;
-    // bf16 copies: the fp32 path's linears, the context projections, the norm and modulation weights
-    DeviceBuffer sa_q, sa_k, sa_v, sa_o, ca_q, ca_o, ca_k, ca_v, mlp1, mlp2;
-    DeviceBuffer sa_qn, sa_kn, ca_qn, ca_kn;
+    // bf16 copies: the fp32 path's linears, the norm and modulation weights
+    DeviceBuffer sa_q, sa_k, sa_v, sa_o, ca_q, ca_o, mlp1, mlp2;
+    DeviceBuffer sa_qn, sa_kn, ca_qn;
     DeviceBuffer mod[6];
 };
 
@@ -123,14 +123,23 @@ void Dit::set_block(int i, const BlockWeights& w) {
     b->sa_o = copy_bf16(w.sa_o, DD, s_, "sa_o");
     b->ca_q = copy_bf16(w.ca_q, DD, s_, "ca_q");
     b->ca_o = copy_bf16(w.ca_o, DD, s_, "ca_o");
-    b->ca_k = copy_bf16(w.ca_k, (size_t)D * C, s_, "ca_k");
-    b->ca_v = copy_bf16(w.ca_v, (size_t)D * C, s_, "ca_v");
+    // the context projections and K norms of all blocks lie one after the other (one product per prompt)
+    if (!ca_kv_all_.get()) {
+        ca_kv_all_.resize((size_t)d_.blocks * 2 * D * C * 2);
+        ca_kn_all_.resize((size_t)d_.blocks * HD * 2);
+    }
+    auto slot = [&](const DeviceBuffer& all, size_t at, const uint16_t* src, size_t n, const char* what) {
+        if (!src) throw std::runtime_error(std::string("missing weight ") + what);
+        ck_hip(hipMemcpyAsync(all.get<uint16_t>() + at, src, n * 2, hipMemcpyDeviceToDevice, s_), what);
+    };
+    slot(ca_kv_all_, (size_t)i * 2 * D * C, w.ca_k, (size_t)D * C, "ca_k");
+    slot(ca_kv_all_, ((size_t)i * 2 + 1) * D * C, w.ca_v, (size_t)D * C, "ca_v");
+    slot(ca_kn_all_, (size_t)i * HD, w.ca_kn, HD, "ca_kn");
     b->mlp1 = copy_bf16(w.mlp1, (size_t)F * D, s_, "mlp1");
     b->mlp2 = copy_bf16(w.mlp2, (size_t)D * F, s_, "mlp2");
     b->sa_qn = copy_bf16(w.sa_qn, HD, s_, "sa_qn");
     b->sa_kn = copy_bf16(w.sa_kn, HD, s_, "sa_kn");
     b->ca_qn = copy_bf16(w.ca_qn, HD, s_, "ca_qn");
-    b->ca_kn = copy_bf16(w.ca_kn, HD, s_, "ca_kn");
     const uint16_t* mods[6] = {w.mod_sa1, w.mod_sa2, w.mod_ca1, w.mod_ca2, w.mod_mlp1, w.mod_mlp2};
     for (int j = 0; j < 6; j++) b->mod[j] = copy_bf16(mods[j], (j % 2 ? 3 * (size_t)D * 256 : 256 * (size_t)D), s_, "mod");
     // the stacked self-attention projection [Wq; Wk; Wv] (one GEMM whose epilogue splits Q, K, V)
@@ -176,23 +185,30 @@ std::unique_ptr<CachedContext> Dit::cache_context(const float* ctx, int real, in
         c->k32.resize((size_t)d_.blocks * real * D * 4);
         c->v32.resize((size_t)d_.blocks * real * D * 4);
     }
+    for (int i = 0; i < d_.blocks; i++)
+        if (!blocks_[i]) throw std::runtime_error("cache_context: block " + std::to_string(i) + " has no weights");
+    // [K | V] = ctx [W_k; W_v]^T of as many blocks at once as 64 MB of fp32 rows hold (a block's own product is too
+    // small to fill the chip and to be worth its launches), then K = rmsnorm(K; ca_kn) in the prepare pass
+    const size_t per = (size_t)2 * D * real * 4;
+    const int group = (int)std::max<size_t>(1, std::min<size_t>(d_.blocks, ((size_t)64 << 20) / per));
     const size_t m = arena_.mark();
-    arena_.reserve(std::max(arena_.capacity(), (size_t)2 * real * D * 4 + 4096));
-    float* k = arena_.f((size_t)real * D);
-    float* v = arena_.f((size_t)real * D);
-    for (int i = 0; i < d_.blocks; i++) {
-        const Block& b = *blocks_.at(i);
-        // K = rmsnorm(ctx W_k^T; ca_kn), V = ctx W_v^T (fp32 products of the bf16 weights)
-        ck(kiln_linear_f32(k, D, ctx, C, b.ca_k.get<uint16_t>(), real, D, C, ks(s_)), "ctx K");
-        ck(kiln_rmsnorm_rows(k, k, b.ca_kn.get<uint16_t>(), real * H, HD, d_.eps, ks(s_)), "ctx K norm");
-        ck(kiln_linear_f32(v, D, ctx, C, b.ca_v.get<uint16_t>(), real, D, C, ks(s_)), "ctx V");
-        ck(kiln_kv_prepare(const_cast<uint16_t*>(c->kv(i)), k, D, v, D, KILN_F32, real, H, nullptr, d_.eps, nullptr,
-                           nullptr, ks(s_)),
+    arena_.reserve(std::max(arena_.capacity(), group * per + 4096));
+    float* kv = arena_.f((size_t)group * 2 * D * real);
+    for (int i = 0; i < d_.blocks; i += group) {
+        const int n = std::min(group, d_.blocks - i), ld = n * 2 * D;
+        ck(kiln_linear_f32(kv, ld, ctx, C, ca_kv_all_.get<uint16_t>() + (size_t)i * 2 * D * C, real, ld, C, ks(s_)),
+           "ctx K/V");
+        ck(kiln_kv_prepare_blocks(const_cast<uint16_t*>(c->kv(i)), kv, ld, n, real, H, ca_kn_all_.get<uint16_t>() + i * HD,
+                                  d_.eps, ks(s_)),
            "ctx K/V prepare");
-        if (fp32) {
-            const size_t n = (size_t)real * D * 4;
-            ck_hip(hipMemcpyAsync(c->k32.get<char>() + n * i, k, n, hipMemcpyDeviceToDevice, s_), "ctx K copy");
-            ck_hip(hipMemcpyAsync(c->v32.get<char>() + n * i, v, n, hipMemcpyDeviceToDevice, s_), "ctx V copy");
+        for (int j = 0; fp32 && j < n; j++) {
+            const size_t row = (size_t)D * 4, at = (size_t)(i + j) * real * D;
+            for (int v = 0; v < 2; v++)
+                ck_hip(hipMemcpy2DAsync((v ? c->v32 : c->k32).get<float>() + at, row, kv + (2 * j + v) * (size_t)D,
+                                        (size_t)ld * 4, row, real, hipMemcpyDeviceToDevice, s_),
+                       "ctx K/V copy");
+            float* k = c->k32.get<float>() + at;
+            ck(kiln_rmsnorm_rows(k, k, ca_kn_all_.get<uint16_t>() + (i + j) * HD, real * H, HD, d_.eps, ks(s_)), "ctx K norm");
         }
     }
     ck_hip(hipStreamSynchronize(s_), "cache_context");

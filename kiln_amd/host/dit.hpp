@@ -188,6 +188,7 @@ class Dit {
     DeviceBuffer t_lin1_, t_lin2_, t_norm_, fmod1_, fmod2_, x_embed_, final_lin_;
     DeviceBuffer mod1_all_, mod2_all_;  // every block's modulation layers stacked (two launches per step)
     bool mods_stacked_ = false;
+    DeviceBuffer ca_kv_all_, ca_kn_all_;  // every block's context projections [W_k; W_v] [2D, ctx_dim] and K norms [128]
     std::vector<std::unique_ptr<Rope>> ropes_;
     Arena arena_;
 };
