@@ -7,8 +7,8 @@
 //
 // Design (gfx950, wave64):
 //  * workgroup = 4 waves x 32 query rows (BM = 128, two workgroups per CU), or 8 waves x 32 rows (one per CU,
-//    for grids whose 256-row tiles fill whole rounds of CUs, or at least one round of units with >= 2048 keys);
-//    K/V stream in half tiles of 32 keys.
+//    for grids whose 256-row tiles fill whole rounds of CUs, or at least one round of units with >= 2048 keys),
+//    or 8 or 4 waves x 16 rows (grids of at most one unit per CU); K/V stream in half tiles of 32 keys.
 //  * scores are computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32_f16 (under the chip's power limit
 //    this shape sustains more flop/s than 32x32x16): a wave's 32 rows are two 16-column query blocks, and
 //    the four lanes n, n+16, n+32, n+48 of a column hold 8 of each half tile's 32 keys, so the row max needs
@@ -122,28 +122,28 @@ struct Chunk8<float> {
     __device__ __forceinline__ float operator[](int e) const { return e < 4 ? a[e] : b[e - 4]; }
 };
 
-// Q tile of one lane: query rows row[qb] (qb = 0, 1: the wave's two 16-row blocks), d chunks {32c + 8g .. +8}
+// Q tile of one lane: query rows row[qb] (qb < QB: the wave's 16-row blocks), d chunks {32c + 8g .. +8}
 // for c = 0..3 (the B operands of S^T = K Q^T), RMSNorm and RoPE applied in fp32, pre-scaled by
 // log2(e)/sqrt(128), rounded once to fp16. The four lanes g = 0..3 of a query column hold its 128 dims.
-template <typename InT, bool QNORM, bool ROPE>
-__device__ __forceinline__ void load_q(const AttnParams& p, const void* q, const int (&row)[2], const bool (&qin)[2],
-                                       int h, int g, half8 (&qreg)[2][4]) {
+template <typename InT, bool QNORM, bool ROPE, int QB>
+__device__ __forceinline__ void load_q(const AttnParams& p, const void* q, const int (&row)[QB], const bool (&qin)[QB],
+                                       int h, int g, half8 (&qreg)[QB][4]) {
     // Every load (Q rows, RoPE rows, norm weights) is issued before any of them is used, unconditionally (rows
     // past Tq read row 0 and are zeroed afterwards): one memory round trip for the whole tile. A per-lane
     // branch around a load, or a conversion scheduled between loads, serializes them.
-    int rr[2];
-    Chunk8<InT> raw[2][4];
+    int rr[QB];
+    Chunk8<InT> raw[QB][4];
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
         rr[qb] = qin[qb] ? row[qb] : 0;
         const InT* qr = reinterpret_cast<const InT*>(q) + (size_t)rr[qb] * p.ldq + h * HD + 8 * g;
 #pragma unroll
         for (int c = 0; c < 4; c++) raw[qb][c].load(qr + 32 * c);
     }
-    floatx4 cr[2][2][2], sr[2][2][2];  // [qb][c < 2][4-element half]: RoPE pairs (d, d + 64) = chunks (c, c + 2)
+    floatx4 cr[QB][2][2], sr[QB][2][2];  // [qb][c < 2][4-element half]: RoPE pairs (d, d + 64) = chunks (c, c + 2)
     if constexpr (ROPE) {
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++)
+        for (int qb = 0; qb < QB; qb++)
 #pragma unroll
             for (int c = 0; c < 2; c++) {
                 const float* cp = p.rcos + (size_t)rr[qb] * 64 + 32 * c + 8 * g;
@@ -166,7 +166,7 @@ __device__ __forceinline__ void load_q(const AttnParams& p, const void* q, const
     // Rows past Tq (which read row 0) are zeroed by the final multiplier; the norm's per-row factor r joins the
     // pre-scale there: q' = RoPE(x * w) * (r * qscale), the same mathematics as RoPE(x * r * w) * qscale.
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
         float x[4][8];
 #pragma unroll
         for (int c = 0; c < 4; c++)
@@ -208,12 +208,13 @@ __device__ __forceinline__ void load_q(const AttnParams& p, const void* q, const
 }
 
 // accumulator item i of key block kb of a 32-key half tile holds key 32*jh + 16*kb + 4*g + i
-__device__ __forceinline__ void mask_half(int jh, int Tk, int g, floatx4 (&a)[2][2]) {
+template <int QB>
+__device__ __forceinline__ void mask_half(int jh, int Tk, int g, floatx4 (&a)[2][QB]) {
     const int kbase = jh * 32 + 4 * g;
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++)
+        for (int qb = 0; qb < QB; qb++)
 #pragma unroll
             for (int i = 0; i < 4; i++)
                 if (kbase + 16 * kb + i >= Tk) a[kb][qb][i] = -INFINITY;
@@ -314,20 +315,21 @@ static_assert(NS == 4, "ring: tiles j-1 (refilled), j, j+1 and j+2 (read this it
 // chip turns into clock).
 // CHAIN: a context chain (one unit per query tile and head, every job in turn); a separate instantiation, so
 // the one-job kernels compile exactly as without the job loop (the loop costs them ~1.5%).
-template <typename InT, typename OutT, bool QNORM, bool ROPE, int NWT, bool CHAIN>
+// QB: 16-row query blocks per wave, 2 or (small grids) 1.
+template <typename InT, typename OutT, bool QNORM, bool ROPE, int NWT, bool CHAIN, int QB>
 __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams p) {  // 2nd: workgroups per CU
     extern __shared__ __attribute__((aligned(16))) _Float16 lds[];  // NS x 16 KB
-    constexpr int KBM = NWT * 32;                          // query rows of the workgroup
+    constexpr int WR = 16 * QB, KBM = NWT * WR;            // query rows of a wave, of the workgroup
     constexpr int KDMA = HT_H * 2 / 16 / (NWT * 64);      // 16-byte DMA pieces per thread per half tile
     static_assert(NWT == 4 || NWT == 8, "4 or 8 waves");
-    constexpr int KNS = NWT == 8 ? NS8 : NS;               // ring stages (half tile j in stage j % KNS)
+    constexpr int KNS = NWT == 8 || QB == 1 ? NS8 : NS;    // ring stages (half tile j in stage j % KNS)
     static_assert(KNS == 4 || KNS == 8, "a power of two: stage = j & (KNS - 1)");
     const int tid = threadIdx.x, lane_in = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g_in = lane_in >> 4;  // 16-lane row of the wave: keys 4g..4g+3 of a key block, dims 8g.. of a d chunk
     Work W;
     if (!decode_work(p, W)) return;
-    half8 qreg[2][4];  // the Q tile (B operands); a context chain keeps it for consecutive jobs of one Q
+    half8 qreg[QB][4];  // the Q tile (B operands); a context chain keeps it for consecutive jobs of one Q
     // one job of the unit: the keys of p.job[jb] for this query tile and head, with its epilogue; qload: load the
     // Q tile (a chain skips it when the job shares the previous job's queries)
     auto run_job = [&](int jb, int lane, int g, bool qload) {
@@ -377,26 +379,26 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 #pragma unroll
     for (int i = 0; i < 3; i++) dma(min(i, nh - 1), i);
     __builtin_amdgcn_sched_barrier(0);
-    int row[2];
-    bool qin[2];
+    int row[QB];
+    bool qin[QB];
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
-        row[qb] = W.qt * KBM + wv * 32 + 16 * qb + (lane & 15);
+    for (int qb = 0; qb < QB; qb++) {
+        row[qb] = W.qt * KBM + wv * WR + 16 * qb + (lane & 15);
         qin[qb] = row[qb] < p.Tq;
     }
-    if (qload) load_q<InT, QNORM, ROPE>(p, J.q, row, qin, W.h, g, qreg);
+    if (qload) load_q<InT, QNORM, ROPE, QB>(p, J.q, row, qin, W.h, g, qreg);
 #pragma unroll
     for (int i = 3; i < KNS - 1; i++) dma(min(i, nh - 1), i);
     KILN_WAIT_VMCNT((KNS - 3) * KDMA);
     __builtin_amdgcn_s_barrier();
 
-    floatx4 o[2][8];  // O^T per query block: d block db holds d = 16*db + 4g + i
-    float m[2], l[2], mx[2];
-    floatx4 sc[2][2], sc2[2][2];  // [key block][query block]: S_j - m and S_{j+1} - m; the unrolled loop
+    floatx4 o[QB][8];  // O^T per query block: d block db holds d = 16*db + 4g + i
+    float m[QB], l[QB], mx[QB];
+    floatx4 sc[2][QB], sc2[2][QB];  // [key block][query block]: S_j - m and S_{j+1} - m; the unrolled loop
                                   // alternates their roles
-    floatx4 mneg[2];              // -m in every item: the first QK MFMA of a chain starts from it
+    floatx4 mneg[QB];              // -m in every item: the first QK MFMA of a chain starts from it
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
 #pragma unroll
         for (int db = 0; db < 8; db++) o[qb][db] = floatx4{0.f, 0.f, 0.f, 0.f};
         l[qb] = 0.f;
@@ -406,7 +408,9 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
     // two MFMAs per half tile instead of eight v_dot2c_f32_f16 on the VALU, which bounds the loop.
     const half8 ones8 = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f,
                          (_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
-    floatx4 lsum[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+    floatx4 lsum[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; qb++) lsum[qb] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     half8 ka[8];  // K operands s = 2c + kb: d chunks 0-1 (s < 4) of the next QK chains are read a phase ahead
 #pragma unroll
@@ -414,14 +418,14 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 #pragma unroll
     for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) sc[kb][qb] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int qb = 0; qb < QB; qb++) sc[kb][qb] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 8; s++)
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) sc[s & 1][qb] = mfma16(ka[s], qreg[qb][s >> 1], sc[s & 1][qb]);
+        for (int qb = 0; qb < QB; qb++) sc[s & 1][qb] = mfma16(ka[s], qreg[qb][s >> 1], sc[s & 1][qb]);
     if (Tk < 32) mask_half(0, Tk, g, sc);
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
         m[qb] = quad_max(max8(sc[0][qb], sc[1][qb]));  // the first half tile sets the running max of the row
         mx[qb] = 0.f;  // max(S_j) - m over this lane's 8 keys of the row (three other lanes hold the rest)
 #pragma unroll
@@ -438,12 +442,13 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
 
     // the running max moves up by d: O and l scale by 2^-d, and S_j - m (cur) shifts by -d
-    auto rescale = [&](floatx4(&cur)[2][2]) {
+    auto rescale = [&](floatx4(&cur)[2][QB]) {
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
-            // the rescale decision is wave-uniform (a ballot over every lane's own maximum), so the row's
-            // common maximum over its four lanes is formed only here, on the rare path
-            const float d = fmaxf(quad_max(mx[qb]), 0.f);
+        for (int qb = 0; qb < QB; qb++) {
+            // the branch is wave-uniform (a ballot over every lane's own maximum), so the row's common maximum over
+            // its four lanes is formed only here, on the rare path; a row moves by its own maximum alone, so its
+            // result does not depend on the rows that share its wave
+            const float qm = quad_max(mx[qb]), d = qm > RESCALE_TH ? qm : 0.f;
             const float corr = __builtin_amdgcn_exp2f(-d);
 #pragma unroll
             for (int db = 0; db < 8; db++) o[qb][db] *= corr;
@@ -458,7 +463,7 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
         }
     };
     auto need_rescale = [&]() {
-        const bool need = fmaxf(mx[0], mx[1]) > RESCALE_TH;
+        const bool need = (QB == 2 ? fmaxf(mx[0], mx[QB - 1]) : mx[0]) > RESCALE_TH;
         return __builtin_amdgcn_ballot_w64(need) != 0;
     };
 
@@ -471,7 +476,7 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
     // workgroups of a CU run in step with each other, and their issue stalls add up there): config 2 kernel
     // -1.5%, config 3 -1%; at the end of the step: config 2 -1.2%. Context chains keep it after the barrier
     // (their short jobs measured +5% with it at the end of the step), and so do 8-wave workgroups (no change).
-    constexpr bool REFILL_LATE = NWT == 4 && !CHAIN;
+    constexpr bool REFILL_LATE = NWT == 4 && !CHAIN && QB == 2;
     auto sync_refill = [&](auto maskn_tag, int j) {
         if constexpr (decltype(maskn_tag)::value) KILN_WAIT_VMCNT(0);
         else KILN_WAIT_VMCNT((KNS - 4) * KDMA);
@@ -480,9 +485,9 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
             dma(min(j + KNS - 1, nh - 1), stage(j + KNS - 1));  // into the stage of tile j-1
     };
     // One half tile j with a successor. MASKN: the successor is the last half tile and ragged.
-    auto step = [&](auto maskn_tag, int j, floatx4 (&cur)[2][2], floatx4 (&sn)[2][2]) {
+    auto step = [&](auto maskn_tag, int j, floatx4 (&cur)[2][QB], floatx4 (&sn)[2][QB]) {
         constexpr bool MASKN = decltype(maskn_tag)::value;
-        if (need_rescale()) rescale(cur);  // lazy rescale (rare)
+        if (__builtin_expect(need_rescale(), 0)) rescale(cur);  // lazy rescale (rare)
         const int st = stage(j), st1 = stage(j + 1);
         half8 va[4];
         {
@@ -499,16 +504,18 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
         // exp/convert work to interleave goes first
         __builtin_amdgcn_s_setprio(1);
         // S_{j+1} on the matrix cores while the VALU turns S_j into P_j: MFMA pair s (d chunk s/2, key block
-        // s%2, both query blocks) with P values 2s, 2s+1 (query block s/4, B-operand elements (2s)%8, +1)
-        half8 pb[2];
+        // s%2, every query block) with P values QB*s .. QB*s + QB - 1 (query block value/8, B-operand element value%8)
+        half8 pb[QB];
 #pragma unroll
         for (int s = 0; s < 8; s++) {
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++)
+            for (int qb = 0; qb < QB; qb++)
                 sn[s & 1][qb] = mfma16(ka[s], qreg[qb][s >> 1], s < 2 ? mneg[qb] : sn[s & 1][qb]);
-            const int qb = s >> 2, e = (2 * s) % 8, kb = e / 4, i = e % 4;
-            pb[qb][e] = (_Float16)__builtin_amdgcn_exp2f(cur[kb][qb][i]);
-            pb[qb][e + 1] = (_Float16)__builtin_amdgcn_exp2f(cur[kb][qb][i + 1]);
+#pragma unroll
+            for (int t = 0; t < QB; t++) {
+                const int qb = (QB * s + t) / 8, e = (QB * s + t) % 8;
+                pb[qb][e] = (_Float16)__builtin_amdgcn_exp2f(cur[e / 4][qb][e % 4]);
+            }
         }
         KILN_FENCE();
 
@@ -529,7 +536,7 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 #pragma unroll
         for (int db = 0; db < 4; db++)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) o[qb][db] = mfma16(va[db], pb[qb], o[qb][db]);
+            for (int qb = 0; qb < QB; qb++) o[qb][db] = mfma16(va[db], pb[qb], o[qb][db]);
         if constexpr (REFILL_LATE && !MASKN) {
             KILN_FENCE();
             dma(min(j + KNS - 1, nh - 1), stage(j + KNS - 1));
@@ -538,11 +545,11 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 #pragma unroll
         for (int db = 0; db < 4; db++)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) o[qb][db + 4] = mfma16(vb[db], pb[qb], o[qb][db + 4]);
+            for (int qb = 0; qb < QB; qb++) o[qb][db + 4] = mfma16(vb[db], pb[qb], o[qb][db + 4]);
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) lsum[qb] = mfma16(ones8, pb[qb], lsum[qb]);
+        for (int qb = 0; qb < QB; qb++) lsum[qb] = mfma16(ones8, pb[qb], lsum[qb]);
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) mx[qb] = max8(sn[0][qb], sn[1][qb]);
+        for (int qb = 0; qb < QB; qb++) mx[qb] = max8(sn[0][qb], sn[1][qb]);
         KILN_FENCE();
     };
 
@@ -557,7 +564,7 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) sc[kb][qb] = sc2[kb][qb];
+            for (int qb = 0; qb < QB; qb++) sc[kb][qb] = sc2[kb][qb];
     };
     int j = 0;
     for (; j + 1 < nplain; j += 2) {
@@ -575,14 +582,14 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
         copy_s();
     }
     // last half tile: no successor
-    if (need_rescale()) rescale(sc);
+    if (__builtin_expect(need_rescale(), 0)) rescale(sc);
     {
         half8 va[8];
         const lds_half8* vp = kptr(stage(j)) + 32 * HD / 8;
 #pragma unroll
         for (int db = 0; db < 8; db++) va[db] = vp[db * 64];
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < QB; qb++) {
             half8 pb;
 #pragma unroll
             for (int e = 0; e < 8; e++) pb[e] = (_Float16)__builtin_amdgcn_exp2f(sc[e / 4][qb][e % 4]);
@@ -593,19 +600,19 @@ __global__ __launch_bounds__(NWT * 64, 8 / NWT) void k_attn_fwd(const AttnParams
     }
     // every row of the ones block holds the full sum: a quarter in each of the four lanes the epilogue adds (exact)
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) l[qb] = lsum[qb][0] * 0.25f;
+    for (int qb = 0; qb < QB; qb++) l[qb] = lsum[qb][0] * 0.25f;
     KILN_WAIT_VMCNT(0);  // drain the re-fetch DMAs before the workgroup's LDS is reused or released
     if (p.ksplit <= 1 && p.store_rows) {
         __builtin_amdgcn_s_barrier();  // every wave is done with the ring: its LDS now stages the output rows
         OutT* stg = reinterpret_cast<OutT*>(lds) + wv * 16 * ORS<OutT>;
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++)
-            epilogue_rows<OutT>(p, J, W.qt * KBM + wv * 32 + 16 * qb, W.h, g, lane, m[qb], l[qb], o[qb], stg);
+        for (int qb = 0; qb < QB; qb++)
+            epilogue_rows<OutT>(p, J, W.qt * KBM + wv * WR + 16 * qb, W.h, g, lane, m[qb], l[qb], o[qb], stg);
         return;
     }
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
-        if (NWT == 4 && p.ksplit > 1) {  // partial result of this key range: unnormalized O, running max m, row sum l
+    for (int qb = 0; qb < QB; qb++) {
+        if (NWT == 4 && QB == 2 && p.ksplit > 1) {  // partial result of this key range: unnormalized O, running max m, row sum l
             const int unit = (W.jb * p.H + W.h) * p.qtiles + W.qt;
             float* po = p.part + (size_t)(unit * p.ksplit + W.ks) * PART_FLOATS;
             const int r = wv * 32 + 16 * qb + (lane & 15);
@@ -859,16 +866,16 @@ size_t attn_split_bytes(int ksplit, int njobs, int Tq, int H) {
     if (ksplit <= 1) return 0;
     return (size_t)((Tq + BM - 1) / BM) * H * njobs * ksplit * PART_FLOATS * sizeof(float);
 }
-template <typename InT, typename OutT, bool QN, bool RP, int NWT, bool CHAIN = false>
+template <typename InT, typename OutT, bool QN, bool RP, int NWT, bool CHAIN = false, int QB = 2>
 static hipError_t launch_nw(AttnParams& p, int Tq, int units, hipStream_t s) {
-    constexpr int KBM = NWT * 32;
+    constexpr int KBM = NWT * 16 * QB;
     p.qtiles = (Tq + KBM - 1) / KBM;
     p.total = p.qtiles * units * p.ksplit;
     const int nb = (p.total + 7) / 8 * 8;
     p.per = nb / 8;
-    auto kern = k_attn_fwd<InT, OutT, QN, RP, NWT, CHAIN>;
+    auto kern = k_attn_fwd<InT, OutT, QN, RP, NWT, CHAIN, QB>;
     // the ring, or the output staging of 16 rows per wave if that is larger (8 waves, fp32 output)
-    const size_t lds = std::max((size_t)(NWT == 8 ? NS8 : NS) * HT_H * sizeof(_Float16), (size_t)NWT * 16 * ORS<OutT> * sizeof(OutT));
+    const size_t lds = std::max((size_t)(NWT == 8 || QB == 1 ? NS8 : NS) * HT_H * sizeof(_Float16), (size_t)NWT * 16 * ORS<OutT> * sizeof(OutT));
     hipLaunchKernelGGL(kern, dim3(nb), dim3(NWT * 64), lds, s, p);
     return hipGetLastError();
 }
@@ -884,9 +891,19 @@ static hipError_t launch_sel(AttnParams p, int Tq, int units, hipStream_t s) {
     for (int i = 0; i < p.njobs; i++) longk &= p.job[i].Tk >= 2048;
     // context chains run 4-wave units: at config 5's cross-attention (432 units of three 512-key contexts) 8-wave
     // units (224 on 256 CUs) measured 62.1 against 58.1 us
+    // Grids of at most one 128-row unit per CU run 16 rows per wave instead of 32: 8 waves to 128 rows, or 4 waves to 64
+    // rows where those still have a CU each, with the 8-stage ring that a CU to itself allows. A lone wave per SIMD
+    // spends most of a step waiting for its own chain of reads, exponentials and products (and, with 4 stages, for
+    // the DMA issued one step earlier); the rows' arithmetic is the same. us per launch, H = 16, fp16 prepared Q, 32 rows
+    // per wave -> 128-row units / 64-row units: T = 256 8.8 -> 7.7 / 6.7, 512 13.0 -> 11.4 / 9.8, 1024 21.8 -> 18.3 / 16.4,
+    // 1536 29.7 -> 26.1 / 40.4 (two rounds), 2048 40.4 -> 37.1; with two rounds of units 2304 52.0 -> 72.1
+    const long u64 = (long)((Tq + 63) / 64) * units, u128 = (long)((Tq + 127) / 128) * units;
+    if (p.chain && u128 <= cus) return launch_nw<InT, OutT, QN, RP, 8, true, 1>(p, Tq, units, s);
     if (p.chain) return launch_nw<InT, OutT, QN, RP, 4, true>(p, Tq, units, s);
     if (p.ksplit <= 1 && cus > 0 && (t8 % cus == 0 || (longk && t8 >= cus)))
         return launch_nw<InT, OutT, QN, RP, 8>(p, Tq, units, s);
+    if (p.ksplit <= 1 && u64 <= cus) return launch_nw<InT, OutT, QN, RP, 4, false, 1>(p, Tq, units, s);
+    if (p.ksplit <= 1 && u128 <= cus) return launch_nw<InT, OutT, QN, RP, 8, false, 1>(p, Tq, units, s);
     hipError_t e = launch_nw<InT, OutT, QN, RP, 4>(p, Tq, units, s);
     if (e != hipSuccess) return e;
     if (p.ksplit > 1) hipLaunchKernelGGL(k_attn_merge<OutT>, dim3(4 * p.qtiles * units), dim3(256), 0, s, p);
