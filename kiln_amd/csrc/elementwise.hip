@@ -429,26 +429,28 @@ __global__ __launch_bounds__(256) void k_exact_attn(float* out, int ldo, const f
 
 // ---- the same for Dh = 128 on the fp32 matrix cores (v_mfma_f32_16x16x4_f32: fp32 products and sums, as the
 // reference's cuBLAS SGEMM fallback computes them) with an online softmax over 32-key tiles ----
-// Workgroup = 4 waves x 32 query rows of one head. Per 16-key block a wave computes S^T = K Q^T for its two 16-row
+// Workgroup = 4 waves x 16*QB query rows of one head. Per 16-key block a wave computes S^T = K Q^T for its QB 16-row
 // query blocks (32 MFMAs each, over d = 32g + s in lane group g and step s) and O^T += V^T P^T (8 d blocks x 4
 // steps): P^T comes straight out of the S^T accumulators (lane group g holds keys 4g + i, i = 0..3, of query
 // lane & 15; step kk takes element kk, and the V^T operand of lane (g, dd) is row 4g + kk of the block at
 // d = 8 dd + db, so the output accumulator db holds d = 32g + 8i + db). K/V tiles are staged in LDS as fp32 with
 // 132-float rows (conflict-free operand reads), two stages.
-constexpr int X_KT = 32, X_RS = 132, X_BM = 128;
+constexpr int X_KT = 32, X_RS = 132;
 constexpr int X_STAGE = 2 * X_KT * X_RS;  // floats: K then V
 
+template <int QB>
 __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, const float* q, int ldq,
                                                           const float* k, int ldk, const float* v, int ldv, int Tq,
                                                           int Tk, int causal, int npad, float scale) {
     extern __shared__ __attribute__((aligned(16))) float xs[];  // 2 stages
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int g = lane >> 4, n = lane & 15;
-    const int h = blockIdx.y, q0 = blockIdx.x * X_BM + wv * 32;
+    constexpr int X_BM = 64 * QB;
+    const int h = blockIdx.y, q0 = blockIdx.x * X_BM + wv * 16 * QB;
     // Q operands: query block qb, row q0 + 16 qb + n, d = 32 g .. 32 g + 31 (rows past Tq read row Tq - 1)
-    float qo[2][32];
+    float qo[QB][32];
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
         const float* qr = q + (size_t)min(q0 + 16 * qb + n, Tq - 1) * ldq + (size_t)h * 128 + 32 * g;
 #pragma unroll
         for (int c = 0; c < 8; c++) {
@@ -487,10 +489,10 @@ __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, c
     // causal: no key past the last query row of the workgroup
     const int kend = causal ? min(Tk, blockIdx.x * X_BM + X_BM) : Tk;
     const int nt = (kend + X_KT - 1) / X_KT;
-    floatx4 o[2][8];
-    float m[2], l[2];
+    floatx4 o[QB][8];
+    float m[QB], l[QB];
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
 #pragma unroll
         for (int db = 0; db < 8; db++) o[qb][db] = floatx4{0.f, 0.f, 0.f, 0.f};
         m[qb] = npad ? 0.f : -INFINITY;  // with padding keys the max starts at their score, 0
@@ -507,7 +509,9 @@ __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, c
         const float* vs = ks + X_KT * X_RS;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
-            floatx4 sc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+            floatx4 sc[QB];
+#pragma unroll
+            for (int qb = 0; qb < QB; qb++) sc[qb] = floatx4{0.f, 0.f, 0.f, 0.f};
             const float* krow = ks + (kb * 16 + n) * X_RS + 32 * g;
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -515,12 +519,12 @@ __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, c
 #pragma unroll
                 for (int e = 0; e < 4; e++)
 #pragma unroll
-                    for (int qb = 0; qb < 2; qb++)
+                    for (int qb = 0; qb < QB; qb++)
                         sc[qb] = __builtin_amdgcn_mfma_f32_16x16x4f32(ka[e], qo[qb][4 * c + e], sc[qb], 0, 0, 0);
             }
-            float pr[2][4];
+            float pr[QB][4];
 #pragma unroll
-            for (int qb = 0; qb < 2; qb++) {
+            for (int qb = 0; qb < QB; qb++) {
                 const int row = q0 + 16 * qb + n;
                 float bm = -INFINITY;
 #pragma unroll
@@ -551,7 +555,7 @@ __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, c
                 const floatx4 va = *reinterpret_cast<const floatx4*>(vrow);
                 const floatx4 vb = *reinterpret_cast<const floatx4*>(vrow + 4);
 #pragma unroll
-                for (int qb = 0; qb < 2; qb++)
+                for (int qb = 0; qb < QB; qb++)
 #pragma unroll
                     for (int db = 0; db < 8; db++)
                         o[qb][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(db < 4 ? va[db] : vb[db - 4], pr[qb][kk],
@@ -564,7 +568,7 @@ __global__ __launch_bounds__(256, 2) void k_exact_attn128(float* out, int ldo, c
         }
     }
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < QB; qb++) {
         float lt = l[qb] + __shfl_xor(l[qb], 16, 64);
         lt += __shfl_xor(lt, 32, 64);
         if (npad) lt += (float)npad * expf(-m[qb]);
@@ -592,8 +596,12 @@ hipError_t launch_exact_attn(float* out, int ldo, const float* q, int ldq, const
     const auto a16 = [](const void* p) { return ((uintptr_t)p % 16) == 0; };
     if (Dh == 128 && Tk > 0 && a16(q) && a16(k) && a16(v) && a16(out) && ldq % 4 == 0 && ldk % 4 == 0 &&
         ldv % 4 == 0 && ldo % 4 == 0) {
-        hipLaunchKernelGGL(k_exact_attn128, dim3((Tq + X_BM - 1) / X_BM, H), dim3(256),
-                           (size_t)2 * X_STAGE * sizeof(float), s, out, ldo, q, ldq, k, ldk, v, ldv, Tq, Tk,
+        // two 64-row workgroups (16 rows per wave) per CU hold up to 512 units; beyond that 32 rows per wave read K and V
+        // half as often. us, H = 16, 128 / 64 rows: T = 256 54 / 34, 1024 208 / 131, 1536 307 / 288, 2048 407 / 381, 3456
+        // 1118 / 1242. A row's sums do not depend on the form.
+        const int qb = (long)((Tq + 63) / 64) * H <= 2L * cu_count() ? 1 : 2;
+        hipLaunchKernelGGL(qb == 1 ? k_exact_attn128<1> : k_exact_attn128<2>, dim3((Tq + 64 * qb - 1) / (64 * qb), H),
+                           dim3(256), (size_t)2 * X_STAGE * sizeof(float), s, out, ldo, q, ldq, k, ldk, v, ldv, Tq, Tk,
                            causal ? 1 : 0, npad, 1.f / sqrtf(128.f));
         return hipGetLastError();
     }

@@ -277,7 +277,6 @@ struct GemmCost {
     double launch, tile, slice, shared;
 };
 double gemm_cost(const GemmCost& c, long tiles, int slices, int cus);
-int cu_count();  // of the current device (256 without one)
 struct SmallGemm {
     int cfg;
     double cost;

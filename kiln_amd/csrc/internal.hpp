@@ -9,6 +9,8 @@ namespace kiln {
 
 enum class DT { F32 = 0, F16 = 1 };
 
+int cu_count();  // CUs of the current device (256 without one)
+
 // One attention problem of a batched launch: queries q (rows [0, Tq), row stride ldq, head h at
 // column h*128) against the prepared K/V buffer kv (Tk real keys, npad analytic zero keys).
 struct AttnJob {

@@ -68,3 +68,17 @@ def test_chain_of_contexts(gpu):
     assert torch.equal(neg, single[2]) and torch.equal(out[T:], single[1])
     kiln_amd.nag_combine(single[0], single[2])
     assert torch.equal(out[:T], single[0])
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_exact_forms_agree_bit_for_bit(gpu, causal):
+    """Exact fp32 attention of 2100 rows (128-row workgroups) against its first 500 rows alone (64-row ones)."""
+    H, T, Tk = 16, 2100, 130
+    g = torch.Generator(device=DEV).manual_seed(4)
+    q, k, v = (torch.randn(t, H * D, device=DEV, generator=g) for t in (T, Tk, Tk))
+    a, b = torch.empty_like(q), torch.empty(500, H * D, device=DEV)
+    kiln_amd.attention_exact(a, q, k, v, T, Tk, H, D, causal=causal, npad=3)
+    kiln_amd.attention_exact(b, q[:500], k, v, 500, Tk, H, D, causal=causal, npad=3)
+    assert torch.equal(a[:500], b)
+    ref = oracle.attn_f64(q[:64].cpu().numpy(), k.cpu().numpy(), v.cpu().numpy(), H, npad=3, causal=causal)
+    assert_close(b[:64].cpu().numpy(), ref, "exact", max_abs=1e-5, mean_abs=1e-6)
