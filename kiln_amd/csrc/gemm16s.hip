@@ -13,8 +13,8 @@
 //    NST - 1 steps ahead; one barrier per step.
 //  * bound by the rate at which a CU takes in operand bytes (30 to 40 B per cycle in every configuration). Measured, us,
 //    one product of M rows with weights from memory, 256-wide tiles -> these: 2048 x 2048 M = 64 36.3 -> 9.3, M = 256
-//    42.9 -> 9.1, M = 1024 45.0 -> 17.5, M = 3072 47.8 -> 35.2; 2048 x 8192 M = 256 131.8 -> 26.9; 8192 x 2048 M = 256
-//    44.5 -> 19.4.
+//    42.9 -> 9.0, M = 1024 45.0 -> 16.7, M = 3072 47.8 -> 35.2; 2048 x 8192 M = 256 131.8 -> 25.3; 8192 x 2048 M = 256
+//    44.5 -> 19.0.
 //  * row-major operands (activations, plain weights) lie in LDS as 128-byte rows of two k slices, 16-byte chunk c
 //    of row r at position c ^ (r & 7): the DMA reads whole 128-byte lines, the operand reads are conflict free.
 //    Prepared weights keep their 64-byte rows (one contiguous run per slice).
@@ -135,26 +135,37 @@ __global__ __launch_bounds__(STHR, 1) void k_gemm16s(const GemmParams p) {
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) acc[nb][mb] = floatx4{0.f, 0.f, 0.f, 0.f};
     // slices s of a stage, s < have
-    auto compute = [&](uint32_t st_base, auto prep_tag, int have) {
+    auto compute = [&](uint32_t st_base, auto prep_tag, int have, auto refill) {
         constexpr bool PREP = decltype(prep_tag)::value;
+        half8 fw[KS][NBW], fa[KS][MB];
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const int s = kg * KS + ks;
             if (s >= have) break;
-            half8 fw[NBW], fa[MB];
 #pragma unroll
             for (int nb = 0; nb < NBW; nb++) {
                 const int row = (nb < 2 ? wrow : wrow_hi) + 16 * nb;
-                fw[nb] = PREP ? read(st_base + s * BN * 64 + row * 64 + ((g ^ ((rl >> 1) & 3)) * 16))
-                              : read(st_base + pair_at(s, BN) + row * 128);
+                fw[ks][nb] = PREP ? read(st_base + s * BN * 64 + row * 64 + ((g ^ ((rl >> 1) & 3)) * 16))
+                                  : read(st_base + pair_at(s, BN) + row * 128);
             }
 #pragma unroll
             for (int mb = 0; mb < MB; mb++)
-                fa[mb] = read(st_base + C::W_BYTES + pair_at(s, BM) + (wm * MB * 16 + mb * 16 + rl) * 128);
+                fa[ks][mb] = read(st_base + C::W_BYTES + pair_at(s, BM) + (wm * MB * 16 + mb * 16 + rl) * 128);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every operand read in flight before the first MFMA waits for one
+        // with k groups (few MFMAs per step) the refill goes behind the reads that the MFMAs wait for: 2048 x 8192, M = 256
+        // 27.6 -> 25.3 us; the 128 x 192 tile keeps it ahead of them (6144 x 2048, M = 3072 95.0, behind them 98.8)
+        if constexpr (KG > 1) {
+            refill();
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (kg * KS + ks >= have) break;
 #pragma unroll
             for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-                for (int nb = 0; nb < NBW; nb++) acc[nb][mb] = mfma16(fw[nb], fa[mb], acc[nb][mb]);
+                for (int nb = 0; nb < NBW; nb++) acc[nb][mb] = mfma16(fw[ks][nb], fa[ks][mb], acc[nb][mb]);
         }
     };
     using Prep = std::integral_constant<bool, WPREP>;
@@ -173,11 +184,14 @@ __global__ __launch_bounds__(STHR, 1) void k_gemm16s(const GemmParams p) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         const int into = stage == 0 ? NST - 1 : stage - 1;
-        if (steady || st + NST - 1 < S) dma(st + NST - 1, into);
+        auto refill = [&]() {
+            if (steady || st + NST - 1 < S) dma(st + NST - 1, into);
+        };
+        if constexpr (KG == 1) refill();
         const uint32_t sb = lds_base + stage * C::STAGE;
-        if (steady) compute(sb, Prep{}, SL);
-        else if (st < S1) compute(sb, Prep{}, KT1 - st * SL);
-        else compute(sb, std::false_type{}, KT2 - (st - S1) * SL);
+        if (steady) compute(sb, Prep{}, SL, refill);
+        else if (st < S1) compute(sb, Prep{}, KT1 - st * SL, refill);
+        else compute(sb, std::false_type{}, KT2 - (st - S1) * SL, refill);
         __builtin_amdgcn_sched_barrier(0);
         stage = stage == NST - 1 ? 0 : stage + 1;
     };
@@ -279,7 +293,10 @@ hipError_t launch_gemm16s(const GemmParams& p, int cfg, int epi, hipStream_t s) 
 // Modelled time of a product in us: a launch, per round of the chip's CUs a tile's fixed cost and its k slices, and
 // the contention of the tiles in flight for L2 and HBM. The coefficients are least-squares fits of measured times
 // (M = 64 .. 6912 x {2048 x 2048, 8192 x 2048, 2048 x 8192, 6144 x 2048}, each configuration at every size, weights
-// rotated through memory): 5 to 10% rms off, and the choice they make costs at most 10% over the best one.
+// rotated through memory), 10 to 18% off at most; the 128 x 128 tile's contention is set above its fit (0.055), where two
+// rounds of it meet the 256-wide tile (2048 x 8192, M = 4096 158 against 151). Over M = 512 .. 4608 of these products with
+// prepared weights the choice then costs at most 3% over the best one. It does not depend on the weight's layout, so a
+// prepared weight gives the bits of the row-major one.
 double gemm_cost(const GemmCost& c, long tiles, int slices, int cus) {
     const double rounds = (double)((tiles + cus - 1) / cus);
     return c.launch + rounds * (c.tile + c.slice * slices) + c.shared * tiles * slices / cus;
@@ -289,11 +306,11 @@ SmallGemm gemm16s_choose(int M, int N, int K, int epi, int cus) {
     static const struct {
         int bn, bm;
         GemmCost c;
-    } cfg[] = {{128, 192, {2.35, 4.67, 0.308, 0.104}},
-               {128, 128, {2.71, 4.82, 0.231, 0.060}},
-               {128, 64, {3.06, 2.09, 0.155, 0.034}},
-               {128, 32, {2.76, 1.25, 0.119, 0.020}},
-               {64, 32, {2.86, 1.61, 0.070, 0.011}}};
+    } cfg[] = {{128, 192, {2.55, 4.76, 0.270, 0.133}},
+               {128, 128, {2.03, 4.75, 0.224, 0.080}},
+               {128, 64, {2.06, 2.97, 0.142, 0.035}},
+               {128, 32, {2.35, 2.09, 0.115, 0.016}},
+               {64, 32, {2.46, 2.05, 0.074, 0.000}}};
     SmallGemm best{-1, 0.0};
     for (int i = 0; i < 5; i++) {
         if (epi == EPI_QKV && cfg[i].bn % 128) continue;

@@ -236,7 +236,7 @@ def test_linear16_prepare_weight_from_bf16(gpu):
 # One shape or two per small-tile configuration (128 x 192, 128 x 128, 128 x 64, 128 x 32, 64 x 32), with a row over or
 # under a tile's edge, a k count that leaves a partial last step (of 2, 4 or 8 slices) and a one-slice LoRA step.
 SMALL = [(2049, 2048, 96, 32), (3000, 2048, 352, 0), (1500, 2048, 352, 32), (1409, 2048, 288, 0), (700, 2048, 288, 32),
-         (257, 6144, 256, 0), (33, 128, 96, 32), (129, 2048, 128, 0), (65, 2048, 2080, 32), (64, 2048, 1312, 0)]
+         (257, 6144, 256, 0), (385, 2048, 320, 32), (33, 128, 96, 32), (129, 2048, 128, 0), (65, 2048, 2080, 32), (64, 2048, 1312, 0)]
 
 
 @pytest.mark.parametrize("T,rows,cols,k2", SMALL)
