@@ -219,9 +219,11 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 if ((__float_as_uint(v[e]) & 0x7fffffffu) > 0x7f800000u && n + e < p.rows) {  // NaN
-                    float s = 0.f;
-                    for (int k = 0; k < p.cols; k++)
-                        s = fmaf(p.x[(size_t)m * p.ldx + k], bf16_to_f32(p.w[(size_t)(n + e) * p.cols + k]), s);
+                    const float* xrow = p.x + (size_t)m * p.ldx;
+                    const uint16_t* wrow = p.w + (size_t)(n + e) * p.cols;
+                    float s = 0.f;  // a NaN stays one: no need to walk the rest of the row
+                    for (int k0 = 0; k0 < p.cols && (__float_as_uint(s) & 0x7fffffffu) <= 0x7f800000u; k0 += 32)
+                        for (int k = k0; k < k0 + 32; k++) s = fmaf(xrow[k], bf16_to_f32(wrow[k]), s);
                     v[e] = s;
                 }
             float* dst = p.y + (size_t)m * p.ldy + n;
