@@ -222,7 +222,9 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
                     const float* xrow = p.x + (size_t)m * p.ldx;
                     const uint16_t* wrow = p.w + (size_t)(n + e) * p.cols;
                     float s = 0.f;  // a NaN stays one: no need to walk the rest of the row
+                    // (unrolled in full, these loops make the code of 256 x 128 tiles 10% slower where no NaN is)
                     for (int k0 = 0; k0 < p.cols && (__float_as_uint(s) & 0x7fffffffu) <= 0x7f800000u; k0 += 32)
+#pragma unroll 4
                         for (int k = k0; k < k0 + 32; k++) s = fmaf(xrow[k], bf16_to_f32(wrow[k]), s);
                     v[e] = s;
                 }
