@@ -65,6 +65,7 @@ const char* kiln_dit_last_error(void);
 int kiln_dit_create(const kiln_dit_dims* dims, kiln_stream_t stream, kiln_dit** out);
 void kiln_dit_destroy(kiln_dit* dit);
 int kiln_dit_set_step_weights(kiln_dit* dit, const kiln_dit_step_weights* w);
+/* Copies block i's weights; a call that fails (a null weight, no memory) leaves the block as it was. */
 int kiln_dit_set_block(kiln_dit* dit, int i, const kiln_dit_block_weights* w);
 
 /* Dit::cache_context: ctx [len, ctx_dim] fp32 device rows, the first `real` real (the rest zero padding, entering

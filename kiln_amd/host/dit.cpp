@@ -123,18 +123,8 @@ void Dit::set_block(int i, const BlockWeights& w) {
     b->sa_o = copy_bf16(w.sa_o, DD, s_, "sa_o");
     b->ca_q = copy_bf16(w.ca_q, DD, s_, "ca_q");
     b->ca_o = copy_bf16(w.ca_o, DD, s_, "ca_o");
-    // the context projections and K norms of all blocks lie one after the other (one product per prompt)
-    if (!ca_kv_all_.get()) {
-        ca_kv_all_.resize((size_t)d_.blocks * 2 * D * C * 2);
-        ca_kn_all_.resize((size_t)d_.blocks * HD * 2);
-    }
-    auto slot = [&](const DeviceBuffer& all, size_t at, const uint16_t* src, size_t n, const char* what) {
-        if (!src) throw std::runtime_error(std::string("missing weight ") + what);
-        ck_hip(hipMemcpyAsync(all.get<uint16_t>() + at, src, n * 2, hipMemcpyDeviceToDevice, s_), what);
-    };
-    slot(ca_kv_all_, (size_t)i * 2 * D * C, w.ca_k, (size_t)D * C, "ca_k");
-    slot(ca_kv_all_, ((size_t)i * 2 + 1) * D * C, w.ca_v, (size_t)D * C, "ca_v");
-    slot(ca_kn_all_, (size_t)i * HD, w.ca_kn, HD, "ca_kn");
+    const DeviceBuffer ca_k = copy_bf16(w.ca_k, (size_t)D * C, s_, "ca_k"), ca_v = copy_bf16(w.ca_v, (size_t)D * C, s_, "ca_v");
+    const DeviceBuffer ca_kn = copy_bf16(w.ca_kn, HD, s_, "ca_kn");
     b->mlp1 = copy_bf16(w.mlp1, (size_t)F * D, s_, "mlp1");
     b->mlp2 = copy_bf16(w.mlp2, (size_t)D * F, s_, "mlp2");
     b->sa_qn = copy_bf16(w.sa_qn, HD, s_, "sa_qn");
@@ -154,7 +144,25 @@ void Dit::set_block(int i, const BlockWeights& w) {
     b->ca_o16 = prep16(b->ca_o.get<uint16_t>(), D, D, s_, "ca_o");
     b->mlp1_16 = prep16(b->mlp1.get<uint16_t>(), F, D, s_, "mlp1");
     b->mlp2_16 = prep16(b->mlp2.get<uint16_t>(), D, F, s_, "mlp2");
-    ck_hip(hipStreamSynchronize(s_), "set_block");  // the stacking buffer goes out of scope
+    // the context projections and K norms of all blocks lie one after the other (one product per prompt). They are
+    // written last, from copies: a call that throws leaves the block that was there whole
+    DeviceBuffer kv_all, kn_all;
+    if (!ca_kv_all_.get()) {
+        kv_all.resize((size_t)d_.blocks * 2 * D * C * 2);
+        kn_all.resize((size_t)d_.blocks * HD * 2);
+    }
+    ck_hip(hipStreamSynchronize(s_), "set_block");
+    if (kv_all.get()) {
+        ca_kv_all_ = std::move(kv_all);
+        ca_kn_all_ = std::move(kn_all);
+    }
+    auto slot = [&](const DeviceBuffer& all, size_t at, const DeviceBuffer& src) {
+        ck_hip(hipMemcpyAsync(all.get<uint16_t>() + at, src.get(), src.bytes(), hipMemcpyDeviceToDevice, s_), "set_block");
+    };
+    slot(ca_kv_all_, (size_t)i * 2 * D * C, ca_k);
+    slot(ca_kv_all_, ((size_t)i * 2 + 1) * D * C, ca_v);
+    slot(ca_kn_all_, (size_t)i * HD, ca_kn);
+    ck_hip(hipStreamSynchronize(s_), "set_block");  // the stacking buffer and the copies go out of scope
     blocks_[i] = std::move(b);
     mods_stacked_ = false;
 }

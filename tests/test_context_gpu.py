@@ -46,6 +46,47 @@ def test_context_groups(gpu, real, fp32):
         assert (got[ref == 0] == 0).all()
 
 
+def _weights(g):
+    bf = lambda o, i: (torch.randn(o, i, device=DEV, generator=g) * i ** -0.5).bfloat16()  # noqa: E731
+    w = {n: bf(D, D) for n in ("sa_q", "sa_k", "sa_v", "sa_o", "ca_q", "ca_o")}
+    w.update(ca_k=bf(D, CTX), ca_v=bf(D, CTX), mlp1=bf(4 * D, D), mlp2=bf(D, 4 * D))
+    w.update({n: (1 + 0.2 * torch.randn(128, device=DEV, generator=g)).bfloat16() for n in ("sa_qn", "sa_kn", "ca_qn", "ca_kn")})
+    w["mod"] = [bf(256, D) if j % 2 == 0 else bf(3 * D, 256) for j in range(6)]
+    return w
+
+
+def test_rejected_set_block_changes_nothing(gpu):
+    """kiln_dit_set_block with a weight missing, whichever: the call fails and the block that was there stays whole (its
+    context projections too, which lie in one allocation with the other blocks'); a first block that fails leaves none."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    d = dit.Dit(2, H, ctx_dim=CTX)
+    old, new = [_weights(g) for _ in range(2)], _weights(g)
+    fields = [f for f, _ in dit.BlockWeights._fields_]
+    flat = dict({k: v for k, v in new.items() if k != "mod"}, **dict(zip(fields[-6:], new["mod"])))
+    ctx = torch.randn(33, CTX, device=DEV, generator=g)
+
+    def reject(missing):
+        w = dit.BlockWeights(*[None if f == missing else flat[f].data_ptr() for f in fields])
+        assert dit.dlib().kiln_dit_set_block(d._h, 0, ctypes.byref(w)) == KILN_EINVAL, missing
+
+    def kv(i):
+        c = d.cache_context(ctx)
+        return torch.as_tensor(_View(c.kv(i), kiln_amd.kv_prepped_bytes(33, H) // 2), device=DEV).clone()
+
+    reject("mlp2")
+    with pytest.raises(kiln_amd.KilnError, match="no weights"):
+        kv(0)
+    for i in range(2):
+        d.set_block(i, **old[i])
+    before = [kv(i) for i in range(2)]
+    for f in fields:
+        reject(f)
+        for i in range(2):
+            assert torch.equal(kv(i), before[i]), f"block {i} after a call without {f}"
+    d.set_block(0, **new)
+    assert not torch.equal(kv(0), before[0]) and torch.equal(kv(1), before[1])
+
+
 def test_kv_prepare_blocks_rejects(gpu):
     L = kiln_amd.lib()
     p = ctypes.c_void_p(256)
