@@ -207,6 +207,10 @@ int kiln_unpatchify(float* latent, const float* tok, int ldt, int Hl, int Wl, ki
  * W bf16 [rows, cols], fp32 arithmetic. */
 int kiln_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols,
                     kiln_stream_t stream);
+/* Which kernel a kiln_linear_f32 call runs, for tests and profiles: the workgroup tile of the bf16 matrix-core form as
+ * (weight rows << 16 | rows of x), 0 for the general form (also for sizes the call refuses). The pointers are only
+ * tested for their alignment. */
+int kiln_linear_f32_tile(const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols);
 /* First-block step cache (engine/src/dit.cu:327-340, used at :404-433): y = a - b (k_sub), and the two sums of
  * the relative L1 change, acc[0] = sum |a - b|, acc[1] = sum |b| (device float[2], overwritten; k_rel_l1). */
 /* Synthetic weights (no reference counterpart: the reference loads checkpoints): p[i] = bf16 of lo + (hi - lo) u_i,

@@ -45,6 +45,7 @@ _SIGS = {
     "kiln_patchify": (_i, [_vp, _vp, _i, _i, _vp]),
     "kiln_unpatchify": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "kiln_linear_f32": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _vp]),
+    "kiln_linear_f32_tile": (_i, [_vp, _i, _vp, _i, _i, _i]),
     "kiln_cfg_combine": (_i, [_vp, _vp, _f, _sz, _vp]),
     "kiln_sub": (_i, [_vp, _vp, _vp, _sz, _vp]),
     "kiln_rel_l1": (_i, [_vp, _vp, _sz, _vp, _vp]),
@@ -437,6 +438,13 @@ def linear_f32(y, x, w_bf16, stream=None):
     _check(lib().kiln_linear_f32(_ptr(y), y.stride(0), _ptr(x), x.stride(0), _ptr(w_bf16), x.shape[0],
                                  w_bf16.shape[0], w_bf16.shape[1], _stream(stream)))
     return y
+
+
+def linear_f32_tile(x, w_bf16):
+    """The kernel that linear_f32 runs for these operands: its workgroup tile (weight rows, rows of x), None for the
+    general form."""
+    t = lib().kiln_linear_f32_tile(_ptr(x), x.stride(0), _ptr(w_bf16), x.shape[0], w_bf16.shape[0], w_bf16.shape[1])
+    return (t >> 16, t & 0xffff) if t else None
 
 
 def cfg_combine(v, vn, cfg, stream=None):

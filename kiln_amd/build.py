@@ -27,12 +27,19 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-fno-honor-nans", "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument",
 ]
+# Sources whose results rest on NaN arithmetic: linear_f32.hip finds by a NaN sum the outputs that it recomputes
+NAN_SOURCES = {"linear_f32.hip"}
+
+
+def flags(src):
+    """hipcc's flags for one source file."""
+    return FLAGS + (["-fhonor-nans"] if src in NAN_SOURCES else [])
 
 
 def _compile(src, where=CSRC):
     out = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
     lang = ["-x", "hip"]
-    cmd = [HIPCC, *lang, *FLAGS, "-c", os.path.join(where, src), "-o", out]
+    cmd = [HIPCC, *lang, *flags(src), "-c", os.path.join(where, src), "-o", out]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")

@@ -793,6 +793,12 @@ int kiln_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* 
                      "linear_f32 launch");
 }
 
+int kiln_linear_f32_tile(const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols) {
+    if (T <= 0 || rows <= 0 || cols <= 0 || !kiln::linear_x3_takes(x, ldx, w_bf16, cols)) return 0;
+    const kiln::LinearTile t = kiln::linear_x3_choose(T, rows, cols);
+    return t.bn << 16 | t.bm;
+}
+
 int kiln_cfg_combine(float* v, const float* vn, float cfg, size_t n, kiln_stream_t stream) {
     kiln::prof::Scope prof_("eltwise", (hipStream_t)stream);
     if (n && (!v || !vn)) return fail(KILN_EINVAL, "cfg_combine: null pointer");

@@ -104,6 +104,10 @@ hipError_t launch_linear_f32(float* y, int ldy, const float* x, int ldx, const u
                              hipStream_t s);
 // the linear layers with cols % 32 == 0 and 16-byte aligned rows (linear_f32.hip); launch_linear_f32 takes all
 bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int cols);
+struct LinearTile {
+    int cfg, bn, bm;  // weight rows and rows of x of the workgroup tile
+};
+LinearTile linear_x3_choose(int T, int rows, int cols);
 hipError_t launch_linear_x3(float* y, int ldy, const float* x, int ldx, const uint16_t* W, int T, int rows, int cols,
                             hipStream_t s);
 hipError_t launch_cfg_combine(float* v, const float* vn, float cfg, size_t n, hipStream_t s);

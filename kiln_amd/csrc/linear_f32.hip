@@ -268,12 +268,7 @@ bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int cols) {
 // here: T = 120, 2048 x 1024 44.9 -> 9.3; T = 1024, 2048 x 2048 92.0 -> 30.6; T = 6912, 8192 x 2048 1840 -> 590 (393
 // TFLOP/s against the 154 of a large fp32 matrix product); T = 6912, 64 x 2048 61.2 -> 15.2. Error against 64 bits
 // (2-norm, K = 2048): 8.1e-7 -> 1.7e-7 to 4.8e-7.
-hipError_t launch_linear_x3(float* y, int ldy, const float* x, int ldx, const uint16_t* W, int T, int rows, int cols,
-                            hipStream_t s) {
-    LinearParams p{};
-    p.y = y, p.x = x, p.w = W;
-    p.ldy = ldy, p.ldx = ldx, p.T = T, p.rows = rows, p.cols = cols;
-    p.vec = ldy % 4 == 0 && ((uintptr_t)y & 15) == 0;
+LinearTile linear_x3_choose(int T, int rows, int cols) {
     static const struct {
         int bn, bm;
         GemmCost c;
@@ -282,14 +277,23 @@ hipError_t launch_linear_x3(float* y, int ldy, const float* x, int ldx, const ui
                {128, 64, {2.13, 2.70, 0.328, 0.070}},
                {128, 32, {1.97, 1.75, 0.200, 0.037}},
                {64, 32, {2.51, 1.90, 0.119, 0.029}}};
-    int best = 0;
+    LinearTile best{};
     double best_cost = 0;
     for (int i = 0; i < 5; i++) {
         const long tiles = (long)((T + cfg[i].bm - 1) / cfg[i].bm) * ((rows + cfg[i].bn - 1) / cfg[i].bn);
         const double t = gemm_cost(cfg[i].c, tiles, cols / 32, cu_count());
-        if (i == 0 || t < best_cost) best = i, best_cost = t;
+        if (i == 0 || t < best_cost) best = {i, cfg[i].bn, cfg[i].bm}, best_cost = t;
     }
-    switch (best) {
+    return best;
+}
+
+hipError_t launch_linear_x3(float* y, int ldy, const float* x, int ldx, const uint16_t* W, int T, int rows, int cols,
+                            hipStream_t s) {
+    LinearParams p{};
+    p.y = y, p.x = x, p.w = W;
+    p.ldy = ldy, p.ldx = ldx, p.T = T, p.rows = rows, p.cols = cols;
+    p.vec = ldy % 4 == 0 && ((uintptr_t)y & 15) == 0;
+    switch (linear_x3_choose(T, rows, cols).cfg) {
         case 0: return launch_x3<X0>(p, s);
         case 1: return launch_x3<X1>(p, s);
         case 2: return launch_x3<X2>(p, s);

@@ -50,21 +50,37 @@ def test_linear_f32_scales(gpu, scale):
     _check(y, x, w)
 
 
-def test_linear_f32_infinities_and_nan(gpu):
-    """The same non-finite outputs as the general form (x one float off its alignment takes it)."""
+# the five tiles: (weight rows, rows of x), and a shape that each takes
+TILES = [((256, 128), (2049, 2050, 96)), ((128, 128), (1025, 2048, 64)), ((128, 64), (500, 2050, 64)),
+         ((128, 32), (96, 128, 64)), ((64, 32), (33, 70, 2080))]
+
+
+@pytest.mark.parametrize("tile,shape", TILES)
+def test_linear_f32_infinities_and_nan(gpu, tile, shape):
+    """The same non-finite outputs as the general form (x one float off its alignment takes it), and every finite output
+    within the bar of its own terms, those beside the recomputed ones too."""
+    T, rows, cols = shape
     g = torch.Generator(device=DEV).manual_seed(2)
-    buf = torch.randn(96 * 64 + 1, device=DEV, generator=g)
-    x = buf[1:].view(96, 64)
-    w = torch.randn(128, 64, device=DEV, generator=g).bfloat16()
+    buf = torch.randn(T * cols + 1, device=DEV, generator=g)
+    x = buf[1:].view(T, cols)
+    w = torch.randn(rows, cols, device=DEV, generator=g).bfloat16()
     x[3, 5], x[7, 0], x[9, 63], x[11, 1] = float("inf"), float("-inf"), float("nan"), 0.0
+    x[T - 1, cols - 1] = float("inf")
     x[20] = 1.0  # no remainders
     w[4, 7], w[6, 1], w[8, 2], w[8, 3] = float("inf"), float("-inf"), float("nan"), 0.0
+    w[rows - 1, cols - 2] = float("-inf")
     x[30, 9] = 3.4e38
-    ya, yb = torch.empty(96, 128, device=DEV), torch.empty(96, 128, device=DEV)
+    ya, yb = torch.empty(T, rows, device=DEV), torch.empty(T, rows, device=DEV)
+    xb = x.clone()
+    assert kiln_amd.linear_f32_tile(x, w) is None and kiln_amd.linear_f32_tile(xb, w) == tile
     kiln_amd.linear_f32(ya, x, w)
-    kiln_amd.linear_f32(yb, x.clone(), w)
+    kiln_amd.linear_f32(yb, xb, w)
     a, b = ya.cpu().numpy(), yb.cpu().numpy()
     assert (np.isnan(a) == np.isnan(b)).all()
     assert (np.isposinf(a) == np.isposinf(b)).all() and (np.isneginf(a) == np.isneginf(b)).all()
-    f = np.isfinite(a)
-    assert np.abs(a[f] - b[f]).max() <= 1e-5 * np.abs(a[f]).max()
+    f = torch.isfinite(ya)
+    xz, wz = (torch.nan_to_num(t.double(), nan=0.0, posinf=0.0, neginf=0.0) for t in (xb, w))
+    ref, bar = xz @ wz.T, cols ** 0.5 * 2.0 ** -21 * (xz.abs() @ wz.abs().T)
+    assert f.float().mean() > 0.7 and f[:, rows - 2].sum() >= T - 6
+    for y in (ya, yb):
+        assert ((y.double() - ref).abs() <= bar)[f].all()
