@@ -5,6 +5,9 @@
 // off by truncation), and a product of two bf16 values is exact in fp32, so x W^T = x1 W^T + x2 W^T + x3 W^T holds
 // term by term: what is left is the rounding of fp32 sums, as in v_mfma_f32_16x16x4_f32, and there are fewer of
 // them. Three v_mfma_f32_16x16x32_bf16 do the work of eight v_mfma_f32_16x16x4_f32 in 3/16 of their cycles.
+// It is 2^24 x that is split, and the sums are scaled back: the last bit of any fp32 value (2^-149) then lies in
+// bf16's normal range, where without the scale the third part of |x| < 2^-110 is cut. (1 to 3% of the time: T = 1024,
+// 2048 x 2048 30.1 -> 30.6 us, x 8192 100.0 -> 102.9; T = 6912, 8192 x 2048 556 -> 560.)
 //
 //  * transposed product (C^T = W x^T): the MFMA's A operand is a 16-row block of W, its B operand 16 rows of x1, x2 or
 //    x3; each lane ends with 4 consecutive output columns of one row.
@@ -13,13 +16,14 @@
 //    tokens or the 64-column final layer still keeps every wave busy.
 //  * W goes global -> LDS by DMA; x through registers, where it is split once per tile, into three bf16 planes in LDS.
 //    Two stages: step s + 1 is split and stored, and step s + 2 of x loaded, while step s is multiplied.
-//  * 0 x inf in a term that fp32 arithmetic would not have (x1 = inf has no remainder; a zero remainder against an
-//    infinite weight) shows as a NaN sum: such an element is recomputed in plain fp32.
+//  * an infinite or NaN sum is recomputed in plain fp32: 2^24 x or its sum past fp32's range (|x| >= 2^104), or 0 x inf
+//    in a term that fp32 arithmetic would not have (a zero remainder against an infinite weight).
 #include "gemm16.hpp"
 
 namespace kiln {
 
 constexpr int XTHR = 512;
+constexpr float X_UP = 0x1p24f, X_DOWN = 0x1p-24f;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
@@ -96,7 +100,7 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
         }
     };
     const uint32_t lds_base = (uint32_t)(size_t)(__attribute__((address_space(3))) char*)smem;
-    // x = x1 + x2 + x3, each the upper half of an fp32 word; 64-byte plane rows, octet c of row r at c ^ ((r >> 1) & 3)
+    // 2^24 x = x1 + x2 + x3, each the upper half of an fp32 word; 64-byte plane rows, octet c of row r at c ^ ((r >> 1) & 3)
     auto split_x = [&](int stage) {
 #pragma unroll
         for (int r = 0; r < X_LD; r++) {
@@ -106,6 +110,7 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
             for (int e = 0; e < 8; e += 2) {
                 uint32_t a[3], b[3];
                 auto cut = [&](float v, uint32_t(&o)[3]) {
+                    v *= X_UP;
 #pragma unroll
                     for (int t = 0; t < 3; t++) {
                         o[t] = __float_as_uint(v);
@@ -215,10 +220,10 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
 #pragma unroll
         for (int nb = 0; nb < NBW; nb++) {
             const int n = n0 + wn * 64 + nb * 16 + 4 * g;
-            floatx4 v = out[nb][j];
+            floatx4 v = out[nb][j] * X_DOWN;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if ((__float_as_uint(v[e]) & 0x7fffffffu) > 0x7f800000u && n + e < p.rows) {  // NaN
+                if ((__float_as_uint(v[e]) & 0x7fffffffu) >= 0x7f800000u && n + e < p.rows) {  // infinite or NaN
                     const float* xrow = p.x + (size_t)m * p.ldx;
                     const uint16_t* wrow = p.w + (size_t)(n + e) * p.cols;
                     float s = 0.f;  // a NaN stays one: no need to walk the rest of the row

@@ -11,6 +11,9 @@ import kiln_amd
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
+# the five tiles: (weight rows, rows of x), and a shape that each takes
+TILES = [((256, 128), (2049, 2050, 96)), ((128, 128), (1025, 2048, 64)), ((128, 64), (500, 2050, 64)),
+         ((128, 32), (96, 128, 64)), ((64, 32), (33, 70, 2080))]
 
 
 def _check(y, x, w, what=""):
@@ -39,20 +42,33 @@ def test_linear_f32_tiles(gpu, T, rows, cols):
     _check(buf[1:T + 1, :rows], wide, w)
 
 
-@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -20, 2.0 ** 100])
+@pytest.mark.parametrize("tile,shape", TILES)
+@pytest.mark.parametrize("exp", [-149, -140, -126, -118, -110, -60, 0, 60, 103, 104, 127])
+def test_linear_f32_split_is_exact(gpu, tile, shape, exp):
+    """A weight with a single 1 in each row picks values of x out: every bit of their 24 has to come through the parts,
+    at both ends of fp32 too (2^-149: subnormal values; 2^104 and up are past the range of the scaled sums)."""
+    T, rows, cols = shape
+    g = torch.Generator(device=DEV).manual_seed(5)
+    n = torch.randint(2 ** 23, 2 ** 24, (T, cols), device=DEV, generator=g) | 1
+    x = torch.ldexp(n.double(), torch.tensor(exp - 23, device=DEV)).float()  # subnormal: fewer bits, rounded here
+    x *= 1 - 2 * torch.randint(0, 2, (T, cols), device=DEV, generator=g).float()
+    pick = torch.randint(0, cols, (rows,), device=DEV, generator=g)
+    w = torch.zeros(rows, cols, device=DEV).index_put_((torch.arange(rows, device=DEV), pick), torch.tensor(1.0, device=DEV)).bfloat16()
+    assert kiln_amd.linear_f32_tile(x, w) == tile
+    y = torch.empty(T, rows, device=DEV)
+    kiln_amd.linear_f32(y, x, w)
+    assert torch.equal(y, x[:, pick]), f"{(y != x[:, pick]).sum().item()} of {y.numel()} differ"
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -120, 2.0 ** -100, 2.0 ** -20, 2.0 ** 100, 2.0 ** 116])
 def test_linear_f32_scales(gpu, scale):
-    """Far from 1 the three parts keep all 24 bits."""
+    """Far from 1 too the sums are as good as fp32's."""
     g = torch.Generator(device=DEV).manual_seed(1)
     x = torch.randn(70, 256, device=DEV, generator=g) * scale
     w = torch.randn(130, 256, device=DEV, generator=g).bfloat16()
     y = torch.empty(70, 130, device=DEV)
     kiln_amd.linear_f32(y, x, w)
     _check(y, x, w)
-
-
-# the five tiles: (weight rows, rows of x), and a shape that each takes
-TILES = [((256, 128), (2049, 2050, 96)), ((128, 128), (1025, 2048, 64)), ((128, 64), (500, 2050, 64)),
-         ((128, 32), (96, 128, 64)), ((64, 32), (33, 70, 2080))]
 
 
 @pytest.mark.parametrize("tile,shape", TILES)
