@@ -264,8 +264,9 @@ static hipError_t launch_x3(LinearParams p, hipStream_t s) {
     return hipGetLastError();
 }
 
+// W's DMA has 32-bit offsets in a tile of up to 256 rows: 256 * cols * 2 bytes below 2 GiB
 bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int cols) {
-    return cols % 32 == 0 && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)W & 15) == 0;
+    return cols % 32 == 0 && cols < (1 << 22) && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)W & 15) == 0;
 }
 
 // The tile with the smallest modelled time (gemm_cost; fitted to measured times of every tile at T = 8 .. 6912 and the

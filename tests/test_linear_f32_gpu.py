@@ -100,3 +100,29 @@ def test_linear_f32_infinities_and_nan(gpu, tile, shape):
     assert f.float().mean() > 0.7 and f[:, rows - 2].sum() >= T - 6
     for y in (ya, yb):
         assert ((y.double() - ref).abs() <= bar)[f].all()
+
+
+def test_linear_f32_rows_past_two_gib(gpu):
+    """64 weight rows of 35 MB: a tile of them is past the 32-bit offsets of the matrix-core form's weight reads, so the
+    call takes the general form. The last rows would lack a third of their terms and more otherwise. One x in a thousand is
+    not 0: sums of n <= 18 000 positive terms, whose relative error is at most n ulp (2^-23) however they are rounded."""
+    cols = 17_500_000 // 32 * 32
+    g = torch.Generator(device=DEV).manual_seed(6)
+    x = torch.zeros(1, cols, device=DEV)
+    x[:, ::1000] = torch.rand(1, (cols + 999) // 1000, device=DEV, generator=g)
+    w = torch.rand(64, cols, device=DEV, generator=g, dtype=torch.bfloat16)
+    y = torch.empty(1, 64, device=DEV)
+    assert kiln_amd.linear_f32_tile(x, w) is None
+    kiln_amd.linear_f32(y, x, w)
+    ref = sum(w[:, c:c + 2 ** 20].double() @ x[0, c:c + 2 ** 20].double() for c in range(0, cols, 2 ** 20))
+    assert ((y[0].double() / ref - 1).abs() <= 18000 * 2.0 ** -23).all()
+
+
+def test_linear_f32_form_limits(gpu):
+    """Which form a call takes at the edges of the matrix-core form's rule (nothing is launched)."""
+    x, w = torch.empty(4, 96, device=DEV), torch.empty(8, 96, device=DEV, dtype=torch.bfloat16)
+    t = lambda xp, ldx, wp, cols: kiln_amd.lib().kiln_linear_f32_tile(xp, ldx, wp, 4, 8, cols)  # noqa: E731
+    px, pw = x.data_ptr(), w.data_ptr()
+    assert t(px, 96, pw, 96) and t(px, 1 << 22, pw, (1 << 22) - 32)
+    assert not t(px, 1 << 22, pw, 1 << 22)
+    assert not t(px, 96, pw, 68) and not t(px, 98, pw, 96) and not t(px + 4, 96, pw, 96) and not t(px, 96, pw + 2, 96)
