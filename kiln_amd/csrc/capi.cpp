@@ -794,7 +794,7 @@ int kiln_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* 
 }
 
 int kiln_linear_f32_tile(const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols) {
-    if (T <= 0 || rows <= 0 || cols <= 0 || !kiln::linear_x3_takes(x, ldx, w_bf16, cols)) return 0;
+    if (T <= 0 || rows <= 0 || cols <= 0 || !kiln::linear_x3_takes(x, ldx, w_bf16, T, rows, cols)) return 0;
     const kiln::LinearTile t = kiln::linear_x3_choose(T, rows, cols);
     return t.bn << 16 | t.bm;
 }

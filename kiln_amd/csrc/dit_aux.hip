@@ -8,7 +8,8 @@
 //   patchify     tok [T, 68] from a 16-channel latent [16, Hl, Wl], 2x2 patches      dit.cu:174-182
 //   unpatchify   latent [16, Hl, Wl] from tok [T, 64]                                dit.cu:184-191
 //   linear_f32   y [T, rows] = x [T, cols] W^T, W bf16 [rows, cols]                 kernels.cu:508-529 (linear; here
-//                the forms whose rows are not whole aligned slices of 32 k: linear_f32.hip takes the others)
+//                the smallest, and the forms whose rows are not whole aligned slices of 32 k: linear_f32.hip takes the
+//                others)
 //   cfg_combine  v = vn + cfg (v - vn)                                              kernels.cu:1058-1062
 #include <algorithm>
 
@@ -410,7 +411,7 @@ hipError_t launch_unpatchify(float* lat, const float* tok, int ldt, int Hl, int 
 }
 hipError_t launch_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* W, int T, int rows, int cols,
                              hipStream_t s) {
-    if (linear_x3_takes(x, ldx, W, cols)) return launch_linear_x3(y, ldy, x, ldx, W, T, rows, cols, s);
+    if (linear_x3_takes(x, ldx, W, T, rows, cols)) return launch_linear_x3(y, ldy, x, ldx, W, T, rows, cols, s);
     const long waves = (long)((T + 15) / 16) * ((rows + 63) / 64);
     hipLaunchKernelGGL(k_linear_f32, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, y, ldy, x, ldx, W, T, rows,
                        cols);

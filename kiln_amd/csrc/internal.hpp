@@ -102,8 +102,9 @@ hipError_t launch_patchify(float* tok, const float* lat, int Hl, int Wl, hipStre
 hipError_t launch_unpatchify(float* lat, const float* tok, int ldt, int Hl, int Wl, hipStream_t s);
 hipError_t launch_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* W, int T, int rows, int cols,
                              hipStream_t s);
-// the linear layers with cols % 32 == 0, cols < 2^22 and 16-byte aligned rows (linear_f32.hip); launch_linear_f32 takes all
-bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int cols);
+// the linear layers with cols % 32 == 0, cols < 2^22 and 16-byte aligned rows, but the smallest (linear_f32.hip);
+// launch_linear_f32 takes all
+bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int T, int rows, int cols);
 struct LinearTile {
     int cfg, bn, bm;  // weight rows and rows of x of the workgroup tile
 };

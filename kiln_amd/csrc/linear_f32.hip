@@ -264,8 +264,14 @@ static hipError_t launch_x3(LinearParams p, hipStream_t s) {
     return hipGetLastError();
 }
 
-// W's DMA has 32-bit offsets in a tile of up to 256 rows: 256 * cols * 2 bytes below 2 GiB
-bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int cols) {
+// W's DMA has 32-bit offsets in a tile of up to 256 rows: 256 * cols * 2 bytes below 2 GiB.
+// One or two slices of k are less than this form's own start and end (LDS, 8 waves, the k groups' merge): k_linear_f32
+// takes them, us, here / there: T = 1, 64 x 32 4.06 / 2.61, 2048 x 32 4.24 / 3.08, 64 x 64 4.14 / 3.41, 2048 x 64 4.26 /
+// 3.98; T = 1000, 64 x 32 4.47 / 3.40, 2048 x 32 6.48 / 5.15; T = 4096, 64 x 64 4.68 / 4.62. Past 2^21 outputs, or at 64
+// columns from a few rows of both on, this form is as fast or faster: T = 2048, 2048 x 32 8.32 / 8.83; T = 16, 2048 x 64
+// 4.25 / 4.39; T = 64, 128 x 64 4.31 / 4.36.
+bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int T, int rows, int cols) {
+    if (cols <= 64 && (size_t)T * rows <= (1 << 21) && (cols <= 32 || rows <= 64 || T <= 4)) return false;
     return cols % 32 == 0 && cols < (1 << 22) && ldx % 4 == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)W & 15) == 0;
 }
 

@@ -27,7 +27,7 @@ def _check(y, x, w, what=""):
 # the five tiles (256 x 128, 128 x 128, 128 x 64, 128 x 32, 64 x 32), a row over and under an edge, rows that end
 # inside a tile and inside a group of four columns, a partial last step of 2, 4 or 8 slices
 @pytest.mark.parametrize("T,rows,cols", [(4097, 2048, 96), (2047, 2048, 352), (1025, 2048, 160), (500, 2050, 288), (65, 129, 64),
-                                         (33, 64, 2080), (1, 3, 32), (6912, 64, 256), (31, 2048, 1056)])
+                                         (33, 64, 2080), (1, 3, 32), (1, 3, 96), (4097, 520, 32), (6912, 64, 256), (31, 2048, 1056)])
 def test_linear_f32_tiles(gpu, T, rows, cols):
     g = torch.Generator(device=DEV).manual_seed(T)
     x = torch.randn(T, cols, device=DEV, generator=g)
@@ -121,8 +121,12 @@ def test_linear_f32_rows_past_two_gib(gpu):
 def test_linear_f32_form_limits(gpu):
     """Which form a call takes at the edges of the matrix-core form's rule (nothing is launched)."""
     x, w = torch.empty(4, 96, device=DEV), torch.empty(8, 96, device=DEV, dtype=torch.bfloat16)
-    t = lambda xp, ldx, wp, cols: kiln_amd.lib().kiln_linear_f32_tile(xp, ldx, wp, 4, 8, cols)  # noqa: E731
+    t = lambda xp, ldx, wp, cols, T=4, rows=8: kiln_amd.lib().kiln_linear_f32_tile(xp, ldx, wp, T, rows, cols)  # noqa: E731
     px, pw = x.data_ptr(), w.data_ptr()
     assert t(px, 96, pw, 96) and t(px, 1 << 22, pw, (1 << 22) - 32)
     assert not t(px, 1 << 22, pw, 1 << 22)
     assert not t(px, 96, pw, 68) and not t(px, 98, pw, 96) and not t(px + 4, 96, pw, 96) and not t(px, 96, pw + 2, 96)
+    # the smallest calls: one slice of k up to 2^21 outputs, two up to 64 weight rows or 4 rows of x
+    assert not t(px, 32, pw, 32, 1024, 2048) and t(px, 32, pw, 32, 1025, 2048)
+    assert not t(px, 64, pw, 64, 4096, 64) and not t(px, 64, pw, 64, 4, 2048)
+    assert t(px, 64, pw, 64, 5, 65) and t(px, 96, pw, 96, 1, 1)
