@@ -80,7 +80,7 @@ __device__ __forceinline__ void stv(_Float16* p, float v) { *p = (_Float16)v; }
 
 // ---- modulated LayerNorm of the DiT block (engine/src/kernels.cu:678-697) ----
 // y = (x - mean) * rsqrt(var + eps) * (1 + scale) + shift, mean and var over the row (two passes, as the
-// reference). A row stays in the registers of a wave (rows of up to 512) or a workgroup: one HBM read, one write.
+// reference). A row stays in the registers of a wave (rows of up to 512, or many of up to 704) or a workgroup: one HBM read, one write.
 __device__ __forceinline__ void st4(float* p, floatx4 v) { *reinterpret_cast<floatx4*>(p) = v; }
 __device__ __forceinline__ void st4(_Float16* p, floatx4 v) {
     half4 h = {(_Float16)v[0], (_Float16)v[1], (_Float16)v[2], (_Float16)v[3]};
@@ -210,7 +210,12 @@ static hipError_t layernorm_mod_sel(OutT* y, const float* x, const float* scale,
                                     float eps, bool vec, hipStream_t s) {
     const dim3 grid((rows + 3) / 4), block(256), grid_rows((rows + 4 * LN_RPW - 1) / (4 * LN_RPW));
     const int nc = dim / 4;
+    // Up to 704 wide and with more than 8 dim rows a wave's 4 rows in turn beat a row to a workgroup, most of whose threads
+    // then hold one chunk or none: us, workgroup / wave form, fp16 out, rows from memory: 6912 x 516 9.14 / 8.21, x 704 9.16 /
+    // 8.76; 16384 x 516 17.7 / 13.5, x 704 18.0 / 16.0. Outside the line: 4096 x 576 6.09 / 6.77, 2304 x 516 4.79 / 6.18,
+    // 16384 x 768 (fp32 out) 20.6 / 22.5.
     if (vec && nc <= 64 * 2) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 2>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
+    else if (vec && nc <= 176 && rows > 8 * dim) hipLaunchKernelGGL((k_layernorm_mod_rows<OutT, 4>), grid_rows, block, 0, s, y, x, scale, shift, rows, dim, eps);
     else if (vec && nc <= 256) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 1>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);
     else if (vec && nc <= 256 * 2) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 2>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);
     else if (vec && nc <= 256 * 4) hipLaunchKernelGGL((k_layernorm_mod_wg<OutT, 4>), dim3(rows), block, 0, s, y, x, scale, shift, rows, dim, eps);

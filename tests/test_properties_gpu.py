@@ -168,7 +168,8 @@ def test_identical_keys_give_mean_value(gpu, Tk):
     assert err <= 2e-4  # |mean| ~ 0.02-0.1: fp16 rounding of the output (<= 2^-14) and fp32 sums of Tk terms
 
 
-@pytest.mark.parametrize("rows,dim", [(1, 512), (3, 516), (2, 1024), (5, 1028), (257, 2048), (2, 2052), (3, 4096), (2, 4100)])
+@pytest.mark.parametrize("rows,dim", [(1, 512), (3, 516), (2, 1024), (5, 1028), (257, 2048), (2, 2052), (3, 4096), (2, 4100),
+                                      (4128, 516), (4129, 516), (5633, 704), (5700, 708)])
 def test_layernorm_mod_row_forms(gpu, rows, dim):
     """The widths on both sides of each row form's edge against a float64 LayerNorm: fp32 rounding of the row's sums
     and of the modulation (a few ulp of the largest term)."""
