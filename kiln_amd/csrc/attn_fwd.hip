@@ -974,7 +974,7 @@ hipError_t launch_kv_prep(const KVPrepJob* jobs, int njobs, DT in, int Tk, int H
     p.Tk = Tk;
     // each block walks two consecutive 32-key half tiles of one head, the second one's loads in flight while
     // the first is converted and stored (measured best at T = 1536 and 4096; one per block for small inputs)
-    const int halves = 2 * kv_tiles(Tk) * H * njobs;
+    const long halves = 2L * kv_tiles(Tk) * H * njobs;
     p.tpb = halves >= 1024 ? 2 : 1;
     p.hpg = hpg > 0 ? hpg : H;
     p.gcols = gcols;

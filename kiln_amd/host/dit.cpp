@@ -198,7 +198,8 @@ std::unique_ptr<CachedContext> Dit::cache_context(const float* ctx, int real, in
     // [K | V] = ctx [W_k; W_v]^T of as many blocks at once as 64 MB of fp32 rows hold (a block's own product is too
     // small to fill the chip and to be worth its launches), then K = rmsnorm(K; ca_kn) in the prepare pass
     const size_t per = (size_t)2 * D * real * 4;
-    const int group = (int)std::max<size_t>(1, std::min<size_t>(d_.blocks, ((size_t)64 << 20) / per));
+    const size_t most = std::min((size_t)64 << 20, per * (65535 / H)) / per;  // a prepare launch takes 65535 heads
+    const int group = (int)std::max<size_t>(1, std::min<size_t>(d_.blocks, most));
     const size_t m = arena_.mark();
     arena_.reserve(std::max(arena_.capacity(), group * per + 4096));
     float* kv = arena_.f((size_t)group * 2 * D * real);
