@@ -55,6 +55,33 @@ def _weights(g):
     return w
 
 
+# one group of three blocks; two blocks and one (12000 tokens)
+@pytest.mark.parametrize("real", [77, 12000])
+def test_context_groups_fp32(gpu, real):
+    """The fp32 K and V of a context of three blocks, which no call hands out: each block run in fp32 against a model of
+    that block alone (whose context is one product of its own; checked against float64 in test_dit_block_gpu.py). The
+    products may run on different tiles, so their sums differ by rounding: 1e-5 of outputs of size 1."""
+    g = torch.Generator(device=DEV).manual_seed(real)
+    ws = [_weights(g) for _ in range(BLOCKS)]
+    d = dit.Dit(BLOCKS, H, ctx_dim=CTX)
+    for i, w in enumerate(ws):
+        d.set_block(i, **w)
+    ctx = torch.randn(real, CTX, device=DEV, generator=g)
+    X0, mods = torch.randn(32, D, device=DEV, generator=g), torch.randn(9 * D, device=DEV, generator=g)
+    c = d.cache_context(ctx, fp32=True)
+    for i, w in enumerate(ws):
+        one = dit.Dit(1, H, ctx_dim=CTX)
+        one.set_block(0, **w)
+        a = d.run_block(i, X0.clone(), mods, 4, 8, [c], fp32=True)
+        b = one.run_block(0, X0.clone(), mods, 4, 8, [one.cache_context(ctx, fp32=True)], fp32=True)
+        assert (a - b).abs().max() <= 1e-5 * max(1.0, b.abs().max().item()), f"block {i}"
+        # the bar tells another block's projections and norm apart
+        for n in ("ca_k", "ca_v", "ca_kn"):
+            one.set_block(0, **dict(w, **{n: ws[(i + 1) % BLOCKS][n]}))
+            z = one.run_block(0, X0.clone(), mods, 4, 8, [one.cache_context(ctx, fp32=True)], fp32=True)
+            assert (z - b).abs().max() > 1e-3, f"block {i} {n}: {(z - b).abs().max().item()}"
+
+
 def test_rejected_set_block_changes_nothing(gpu):
     """kiln_dit_set_block with a weight missing, whichever: the call fails and the block that was there stays whole (its
     context projections too, which lie in one allocation with the other blocks'); a first block that fails leaves none."""
