@@ -33,10 +33,21 @@ def test_small_grid(gpu, H, Tq, Tk, npad):
                 assert torch.isnan(buf[:off]).all() and torch.isnan(buf[off + Tq * ld:]).all()
 
 
-@pytest.mark.parametrize("T", [256, 1100, 1536])
-def test_forms_agree_bit_for_bit(gpu, T):
-    """One item (64- or 128-row units of 16-row waves) against the same item in a batch of four (32-row waves), with
-    maxima that move late in the row, so that rows of one wave rescale at different steps."""
+def _form(T, Tk, units):
+    """The kernel form of a launch (waves x query rows of a wave) by the launcher's rule, units = items x heads."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    u64, u128, t8 = ((T + n - 1) // n * units for n in (64, 128, 256))
+    if t8 % cus == 0 or (Tk >= 2048 and t8 >= cus):
+        return "8x32"
+    return "4x16" if u64 <= cus else "8x16" if u128 <= cus else "4x32"
+
+
+@pytest.mark.parametrize("T,alone,four_items", [(700, "4x16", "4x32"), (1000, "4x16", "8x32"), (1100, "8x16", "4x32"),
+                                                (1536, "8x16", "4x32"), (2048, "8x16", "8x32")])
+def test_forms_agree_bit_for_bit(gpu, T, alone, four_items):
+    """One item (64- or 128-row units of 16-row waves) against the same item in a batch of four (32-row waves, 4 or 8 of
+    them), with maxima that move late in the row, so that rows of one wave rescale at different steps."""
+    assert (_form(T, T, 16), _form(T, T, 64)) == (alone, four_items)
     H = 16
     g = torch.Generator(device=DEV).manual_seed(T)
     q, k, v = (torch.randn(T, H * D, device=DEV, generator=g) for _ in range(3))
