@@ -181,6 +181,11 @@ int kiln_linear16_prepped(void* y, int ldy, const uint16_t* x16, int T, const ui
                           int epi, const float* gate, float beta, const uint16_t* a2, const uint16_t* w2, int k2,
                           kiln_stream_t stream);
 
+/* Which workgroup tile a kiln_linear16 call of these sizes runs on, plain or prepared (weight rows << 16 | rows of x16), for
+ * tests and profiles; 0 for sizes that the call refuses. epi 4: the projection inside kiln_dit_self_attn_x16 (rows = 3 D)
+ * and kiln_dit_cross_attn_x16 (rows = D). */
+int kiln_linear16_tile(int T, int rows, int cols, int epi, int k2);
+
 /* ---- the DiT forward's passes around the transformer blocks (engine/src/dit.cu:242-272, 414-417, 537-545) ---- */
 
 /* Replaces matvec() (engine/src/gpu.h:122, kernels.cu k_matvec): y[r] = sum_c W[r][c] x[c] (+ add[r]), W bf16

@@ -45,6 +45,7 @@ _SIGS = {
     "kiln_patchify": (_i, [_vp, _vp, _i, _i, _vp]),
     "kiln_unpatchify": (_i, [_vp, _vp, _i, _i, _i, _vp]),
     "kiln_linear_f32": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _vp]),
+    "kiln_linear16_tile": (_i, [_i, _i, _i, _i, _i]),
     "kiln_linear_f32_tile": (_i, [_vp, _i, _vp, _i, _i, _i]),
     "kiln_cfg_combine": (_i, [_vp, _vp, _f, _sz, _vp]),
     "kiln_sub": (_i, [_vp, _vp, _vp, _sz, _vp]),
@@ -376,6 +377,13 @@ class PreppedWeight:
 
     def is_contiguous(self):
         return True
+
+
+def linear16_tile(T, rows, cols, epi=KILN_EPI_F32, k2=0):
+    """The workgroup tile (weight rows, rows of x16) that linear16 runs these sizes on; epi 4: the fused sections'
+    projections."""
+    t = lib().kiln_linear16_tile(T, rows, cols, epi, k2)
+    return t >> 16, t & 0xffff
 
 
 def linear16(y, x16, w16, epi=KILN_EPI_F32, gate=None, beta=0.0, a2=None, w2=None, stream=None):

@@ -719,6 +719,13 @@ int kiln_linear16_prepped(void* y, int ldy, const uint16_t* x16, int T, const ui
     return linear16_impl("linear16_prepped", y, ldy, x16, T, wp, rows, cols, epi, gate, beta, a2, w2, k2, true, stream);
 }
 
+int kiln_linear16_tile(int T, int rows, int cols, int epi, int k2) {
+    if (T <= 0 || rows <= 0 || cols <= 0 || k2 < 0 || rows % 128 || cols % 32 || k2 % 32 || epi < KILN_EPI_F32 || epi > kiln::EPI_QKV)
+        return 0;
+    const kiln::GemmTile t = kiln::gemm16_choose(T, rows, cols + k2, epi);
+    return t.bn << 16 | t.bm;
+}
+
 size_t kiln_linear16_prepped_weight_bytes(int rows, int cols) {
     if (rows <= 0 || cols <= 0) return 0;
     return kiln::gemm16_prepped_bytes(rows, cols);

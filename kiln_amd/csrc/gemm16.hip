@@ -375,6 +375,19 @@ static int gemm16_mb(int M, int N, int cus, long* tiles) {
     return best;
 }
 
+// Few rows leave most CUs without a 256-wide tile: M = 256 x 2048 x 2048 takes 42.9 us on this kernel's 16 tiles
+// and 9.0 us on 64 x 32 ones, M = 1024 45.0 against 16.8 (128 x 64), M = 3072 49.3 against 35.5 (128 x 192); at
+// M = 4608 it is 54.0 against 72.5. The models meet near the size where the large tiles fill the chip.
+GemmTile gemm16_choose(int M, int N, int K, int epi) {
+    const int cus = cu_count();
+    long tiles = 0;
+    const int mb = gemm16_mb(M, N, cus, &tiles);
+    const SmallGemm small = gemm16s_choose(M, N, K, epi, cus);
+    const double large = gemm_cost({1.54, 1.57 * mb, 0.0663 * mb, 0.0315 * mb}, tiles, K / GBK, cus);
+    if (small.cost < large) return {small.cfg, small.bn, small.bm};
+    return {-1, GBN, 32 * mb};
+}
+
 hipError_t launch_gemm16(const GemmLaunch& g, hipStream_t s) {
     GemmParams p;
     p.a = reinterpret_cast<const _Float16*>(g.a);
@@ -404,16 +417,9 @@ hipError_t launch_gemm16(const GemmLaunch& g, hipStream_t s) {
         p.rcos = g.rcos;
         p.rsin = g.rsin;
     }
-    // Few rows leave most CUs without a 256-wide tile: M = 256 x 2048 x 2048 takes 42.9 us on this kernel's 16 tiles
-    // and 9.0 us on 64 x 32 ones, M = 1024 45.0 against 16.8 (128 x 64), M = 3072 49.3 against 35.5 (128 x 192); at
-    // M = 4608 it is 54.0 against 72.5. The models meet near the size where the large tiles fill the chip.
-    const int cus = cu_count();
-    long tiles = 0;
-    const int mb = gemm16_mb(g.M, g.N, cus, &tiles);
-    const SmallGemm small = gemm16s_choose(g.M, g.N, g.K + g.K2, g.epi, cus);
-    const double large = gemm_cost({1.54, 1.57 * mb, 0.0663 * mb, 0.0315 * mb}, tiles, (g.K + g.K2) / GBK, cus);
-    if (small.cost < large) return launch_gemm16s(p, small.cfg, g.epi, s);
-    if (mb == 7) return launch_mb<7>(p, g.epi, s);
+    const GemmTile t = gemm16_choose(g.M, g.N, g.K + g.K2, g.epi);
+    if (t.cfg >= 0) return launch_gemm16s(p, t.cfg, g.epi, s);
+    if (t.bm == 224) return launch_mb<7>(p, g.epi, s);
     return launch_mb<8>(p, g.epi, s);
 }
 

@@ -51,7 +51,6 @@ struct GemmParams {
     const float* rcos;  // [T, 64]
     const float* rsin;
 };
-constexpr int EPI_QKV = 4;
 __device__ __forceinline__ floatx4 mfma16(half8 a, half8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
@@ -280,6 +279,7 @@ double gemm_cost(const GemmCost& c, long tiles, int slices, int cus);
 struct SmallGemm {
     int cfg;
     double cost;
+    int bn, bm;
 };
 SmallGemm gemm16s_choose(int M, int N, int K, int epi, int cus);
 hipError_t launch_gemm16s(const GemmParams& p, int cfg, int epi, hipStream_t s);

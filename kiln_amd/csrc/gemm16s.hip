@@ -311,12 +311,12 @@ SmallGemm gemm16s_choose(int M, int N, int K, int epi, int cus) {
                {128, 64, {2.06, 2.97, 0.142, 0.035}},
                {128, 32, {2.35, 2.09, 0.115, 0.016}},
                {64, 32, {2.46, 2.05, 0.074, 0.000}}};
-    SmallGemm best{-1, 0.0};
+    SmallGemm best{-1, 0.0, 0, 0};
     for (int i = 0; i < 5; i++) {
         if (epi == EPI_QKV && cfg[i].bn % 128) continue;
         const long tiles = (long)((M + cfg[i].bm - 1) / cfg[i].bm) * (N / cfg[i].bn);
         const double t = gemm_cost(cfg[i].c, tiles, K / GBK, cus);
-        if (best.cfg < 0 || t < best.cost) best = {i, t};
+        if (best.cfg < 0 || t < best.cost) best = {i, t, cfg[i].bn, cfg[i].bm};
     }
     return best;
 }

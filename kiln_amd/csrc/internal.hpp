@@ -59,6 +59,7 @@ struct KVPrepJob {
 hipError_t launch_kv_prep(const KVPrepJob* jobs, int njobs, DT in, int Tk, int H, const uint16_t* kw, float eps,
                           const float* rcos, const float* rsin, hipStream_t s, int hpg = 0, int gcols = 0);
 
+constexpr int EPI_QKV = 4;  // after kiln_epi's
 // acc = a [M,K] w[N,K]^T (+ a2 [M,K2] w2[N,K2]^T), all fp16 dense rows; epilogue `epi` (kiln_epi) into c (row
 // stride ldc). N % 128 == 0, K % 32 == 0, K2 % 32 == 0, 16-byte aligned operand bases.
 struct GemmLaunch {
@@ -75,7 +76,7 @@ struct GemmLaunch {
     int M, N;
     int epi;
     bool wprep;  // w in the prepared layout of launch_gemm_wprep
-    // epi == 4 (the DiT self-attention projection, N = 3 * 128 * H, H even): Q rows and prepared K/V per item
+    // EPI_QKV (the DiT self-attention projection, N = 3 * 128 * H, H even): Q rows and prepared K/V per item
     uint16_t* q16;
     uint16_t* kvp[MAX_JOBS];
     int T, H;
@@ -88,6 +89,12 @@ struct GemmLaunch {
 // zero the last (partial) 64-key tile of each item's and head's prepared K/V before a projection writes the keys
 hipError_t launch_kv_zero_tail(uint16_t* const* kvp, int njobs, int T, int H, hipStream_t s);
 hipError_t launch_gemm16(const GemmLaunch& g, hipStream_t s);
+// the workgroup tile that a product takes (K with the LoRA's K2): bn weight rows x bm activation rows, cfg the small-tile
+// kernel's configuration or -1 for the large tile
+struct GemmTile {
+    int cfg, bn, bm;
+};
+GemmTile gemm16_choose(int M, int N, int K, int epi);
 // Weight [N, K] (fp16, or bf16 converted as the reference's weight_to_f16) into the prepared tile layout.
 size_t gemm16_prepped_bytes(int N, int K);
 hipError_t launch_gemm_wprep(uint16_t* wp, const uint16_t* w, int N, int K, bool src_bf16, hipStream_t s);

@@ -314,13 +314,7 @@ def test_step_cache_skip_reuses_residual(gpu):
     np.testing.assert_array_equal(y.cpu().numpy(), (a - b).numpy())
 
 
-@pytest.mark.parametrize("Hh,Hp_,Wp_,Bb", [(4, 8, 12, 2), (2, 10, 10, 3), (16, 48, 72, 2), (16, 32, 60, 2)])
-def test_dit_self_attn_x16_fused_projection(gpu, Hh, Hp_, Wp_, Bb):
-    """kiln_dit_self_attn_x16 (QKV GEMM whose epilogue does QK-RMSNorm, RoPE and the K/V preparation) against
-    the float64 statement of dit.cu:460-469 on sampled rows (BASELINE bar: max-abs 2e-3, mean-abs 2e-4), and
-    against the unfused path (linear16 F32 + kiln_dit_self_attn_fused) on every output. T = 100 has a partial
-    last key tile; T = 3456 x 16 heads is config 5's shape; T = 1920 x 16 heads x 2 items gives 256 query tiles
-    of 256 rows, which on a 256-CU part selects the 8-wave attention kernel for both paths."""
+def _check_self_attn_x16(Hh, Hp_, Wp_, Bb):
     Dd, Tt = Hh * HD, Hp_ * Wp_
     g = torch.Generator().manual_seed(34 + Hh)
     x = (torch.randn(Bb * Tt, Dd, generator=g)).half()
@@ -351,6 +345,27 @@ def test_dit_self_attn_x16_fused_projection(gpu, Hh, Hp_, Wp_, Bb):
         errs.append((out[b * Tt:(b + 1) * Tt][sel.to(DEV)].cpu().double() - ref).abs())
     e = torch.cat(errs)
     assert e.max().item() <= 2e-3 and e.mean().item() <= 2e-4, (e.max().item(), e.mean().item())
+
+
+@pytest.mark.parametrize("Hh,Hp_,Wp_,Bb", [(4, 8, 12, 2), (2, 10, 10, 3), (16, 48, 72, 2), (16, 32, 60, 2)])
+def test_dit_self_attn_x16_fused_projection(gpu, Hh, Hp_, Wp_, Bb):
+    """kiln_dit_self_attn_x16 (QKV GEMM whose epilogue does QK-RMSNorm, RoPE and the K/V preparation) against
+    the float64 statement of dit.cu:460-469 on sampled rows (BASELINE bar: max-abs 2e-3, mean-abs 2e-4), and
+    against the unfused path (linear16 F32 + kiln_dit_self_attn_fused) on every output. T = 100 has a partial
+    last key tile; T = 3456 x 16 heads is config 5's shape; T = 1920 x 16 heads x 2 items gives 256 query tiles
+    of 256 rows, which on a 256-CU part selects the 8-wave attention kernel for both paths."""
+    _check_self_attn_x16(Hh, Hp_, Wp_, Bb)
+
+
+# The tiles of the fused Q/K/V product (weight rows, rows), each with whole 32-key half tiles per item (V leaves through
+# LDS) and with T % 32 != 0 (V scatters, items meet inside a tile)
+@pytest.mark.parametrize("tile,Hh,Hp_,Wp_,Bb", [
+    ((128, 32), 2, 8, 8, 2), ((128, 32), 2, 10, 10, 2), ((128, 64), 2, 24, 32, 2), ((128, 64), 2, 25, 28, 2),
+    ((128, 128), 2, 32, 48, 2), ((128, 128), 2, 30, 50, 2), ((128, 192), 4, 32, 32, 3), ((128, 192), 4, 30, 30, 3),
+    ((256, 224), 4, 40, 48, 3), ((256, 224), 4, 50, 70, 2), ((256, 256), 4, 48, 72, 3), ((256, 256), 4, 50, 70, 3)])
+def test_dit_self_attn_x16_every_projection_tile(gpu, tile, Hh, Hp_, Wp_, Bb):
+    assert kiln_amd.linear16_tile(Bb * Hp_ * Wp_, 3 * Hh * HD, Hh * HD, epi=4) == tile
+    _check_self_attn_x16(Hh, Hp_, Wp_, Bb)
 
 
 def test_dit_cross_attn_x16_fused_projection(gpu):

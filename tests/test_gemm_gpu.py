@@ -233,35 +233,46 @@ def test_linear16_prepare_weight_from_bf16(gpu):
     _check(oracle.EPI_F32, y.cpu().double().numpy(), ref.astype(np.float64), _abs_acc(x, w16), cols)
 
 
-# One shape or two per small-tile configuration (128 x 192, 128 x 128, 128 x 64, 128 x 32, 64 x 32), with a row over or
-# under a tile's edge, a k count that leaves a partial last step (of 2, 4 or 8 slices) and a one-slice LoRA step.
-SMALL = [(2049, 2048, 96, 32), (3000, 2048, 352, 0), (1500, 2048, 352, 32), (1409, 2048, 288, 0), (700, 2048, 288, 32),
-         (257, 6144, 256, 0), (385, 2048, 320, 32), (33, 128, 96, 32), (129, 2048, 128, 0), (65, 2048, 2080, 32), (64, 2048, 1312, 0)]
+# One shape or two per small-tile configuration, with a row over or under a tile's edge, a k count that leaves a partial
+# last step (of 2, 4 or 8 slices) and a one-slice LoRA step; then the tile (weight rows, activation rows) that takes it
+SMALL = [(2049, 2048, 96, 32, (128, 192)), (3000, 2048, 352, 0, (128, 192)), (1500, 2048, 352, 32, (128, 128)),
+         (1409, 2048, 288, 0, (128, 128)), (700, 2048, 288, 32, (128, 64)), (257, 6144, 256, 0, (128, 64)),
+         (385, 2048, 320, 32, (128, 32)), (33, 128, 96, 32, (64, 32)), (129, 2048, 128, 0, (64, 32)),
+         (65, 2048, 2080, 32, (64, 32)), (64, 2048, 1312, 0, (64, 32))]
+# The large tiles at both heights: ragged rows, one to four k tiles (fewer than the ring's stages, and as many), LoRA pairs
+# of one and two k tiles, a half-empty last column tile (rows % 256 == 128)
+LARGE = [(6913, 2048, 96, 32, (256, 224)), (4100, 2176, 352, 32, (256, 224)), (6912, 1920, 128, 64, (256, 224)),
+         (6913, 2176, 96, 32, (256, 256)), (7001, 2176, 64, 64, (256, 256)), (7000, 2176, 32, 0, (256, 256))]
 
 
-@pytest.mark.parametrize("T,rows,cols,k2", SMALL)
-def test_linear16_small_tiles(gpu, T, rows, cols, k2):
-    """Every epilogue of the small tiles on up to 96 sampled rows against the oracle (the first, the last and the
-    rows around them among them), plain and prepared weights bit for bit alike. The module's bar holds: the k
-    groups' sums are fp32 sums of another order."""
+def _every_epilogue(T, rows, cols, k2, tile, pairs=False):
+    """Every epilogue on up to 96 sampled rows against the oracle (the first, the last and the rows around them among
+    them), plain and prepared weights bit for bit alike. pairs: rows of rows + 6 elements, 2 elements into the buffer, so
+    that outputs leave in pairs; what lies around them stays untouched. The module's bar holds: the k groups' sums are
+    fp32 sums of another order."""
     gen = torch.Generator().manual_seed(11)
     x, w = _f16(gen, (T, cols)), _f16(gen, (rows, cols), cols ** -0.5)
     a2, w2 = (_f16(gen, (T, k2)), _f16(gen, (rows, k2), 0.1)) if k2 else (None, None)
     gate = torch.randn(rows, generator=gen)
     idx = torch.unique(torch.cat([torch.arange(min(T, 33)), torch.randperm(T, generator=gen)[:30], torch.arange(max(0, T - 33), T)]))
-    wd = w.to(DEV)
+    xd, wd = x.to(DEV), w.to(DEV)
     wp = kiln_amd.linear16_prepare_weight(wd)
+    off, ld = (2, rows + 6) if pairs else (0, rows)
     for epi in EPIS:
+        assert kiln_amd.linear16_tile(T, rows, cols, epi, k2) == tile
         fp32_out = epi in (oracle.EPI_F32, oracle.EPI_RESID)
         y0 = torch.randn((T, rows), generator=gen).to(torch.float32 if fp32_out else torch.float16)
-        g = gate if epi == oracle.EPI_RESID else None
+        g = gate if epi == oracle.EPI_RESID and not pairs else None
         beta = 0.5 if epi == oracle.EPI_F32 else 0.0
         out = []
         for weight in (wd, wp):
-            y = y0.to(DEV)
-            kiln_amd.linear16(y, x.to(DEV), weight, epi=epi, gate=g.to(DEV) if g is not None else None, beta=beta,
+            buf = torch.full((off + T * ld,), float("nan"), dtype=y0.dtype, device=DEV)
+            y = buf[off:].view(T, ld)[:, :rows]
+            y.copy_(y0)
+            kiln_amd.linear16(y, xd, weight, epi=epi, gate=g.to(DEV) if g is not None else None, beta=beta,
                               a2=a2.to(DEV) if k2 else None, w2=w2.to(DEV) if k2 else None)
-            out.append(y)
+            assert torch.isnan(buf[:off]).all() and torch.isnan(buf[off:].view(T, ld)[:, rows:]).all()
+            out.append(y.contiguous())
         assert torch.equal(out[0].view(torch.uint8), out[1].view(torch.uint8)), f"epi {epi}"
         ref = oracle.linear16(_bits(x[idx]), _bits(w), epi, y=y0[idx].numpy() if fp32_out else None,
                               gate=g.numpy() if g is not None else None, beta=beta,
@@ -270,3 +281,18 @@ def test_linear16_small_tiles(gpu, T, rows, cols, k2):
             ref = ref.view(np.float16)
         _check(epi, out[0].cpu()[idx].double().numpy(), ref.astype(np.float64),
                _abs_acc(x[idx], w, a2[idx] if k2 else None, w2), cols + k2, g.numpy() if g is not None else None)
+
+
+@pytest.mark.parametrize("T,rows,cols,k2,tile", SMALL)
+def test_linear16_small_tiles(gpu, T, rows, cols, k2, tile):
+    _every_epilogue(T, rows, cols, k2, tile)
+
+
+@pytest.mark.parametrize("T,rows,cols,k2,tile", LARGE + SMALL[::2])
+def test_linear16_pair_stores_of_every_tile(gpu, T, rows, cols, k2, tile):
+    _every_epilogue(T, rows, cols, k2, tile, pairs=True)
+
+
+@pytest.mark.parametrize("T,rows,cols,k2,tile", LARGE)
+def test_linear16_large_tiles(gpu, T, rows, cols, k2, tile):
+    _every_epilogue(T, rows, cols, k2, tile)
