@@ -77,6 +77,44 @@ __device__ __forceinline__ float gelu_erf(float v) {
 }
 
 
+// Small tiles (gemm16s.hip, linear_f32.hip): consecutive workgroups of an XCD share a weight tile in its L2. Tile i of an
+// XCD-contiguous range lies in a raster group of `group` row tiles, column by column.
+__device__ __forceinline__ void raster_tile(int i, int group, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int per_group = group * tiles_n, g0 = (i / per_group) * group, gsz = min(group, tiles_m - g0);
+    tm = g0 + (i % per_group) % gsz, tn = (i % per_group) / gsz;
+}
+// The accumulators of a workgroup's KG groups of MN waves meet in LDS (every wave's blocks, any stage's memory), in the
+// groups' order; group kg ends with row blocks kg, kg + KG, .. of its wave position.
+template <int MN, int MB, int KG>
+__device__ __forceinline__ void merge_k_groups(const floatx4 (&acc)[NBW][MB], floatx4 (&out)[NBW][(MB + KG - 1) / KG],
+                                               floatx4* red, int wv, int kg, int lane) {
+    constexpr int MBO = (MB + KG - 1) / KG;
+    if constexpr (KG == 1) {
+#pragma unroll
+        for (int nb = 0; nb < NBW; nb++)
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) out[nb][mb] = acc[nb][mb];
+    } else {
+        __syncthreads();  // every wave is done with the stages
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int nb = 0; nb < NBW; nb++) red[((wv * MB + mb) * NBW + nb) * 64 + lane] = acc[nb][mb];
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < MBO; j++) {
+            const int mb = min(kg + KG * j, MB - 1);
+#pragma unroll
+            for (int nb = 0; nb < NBW; nb++) {
+                floatx4 t = red[(((wv % MN) * MB + mb) * NBW + nb) * 64 + lane];
+#pragma unroll
+                for (int k = 1; k < KG; k++) t += red[(((k * MN + wv % MN) * MB + mb) * NBW + nb) * 64 + lane];
+                out[nb][j] = t;
+            }
+        }
+    }
+}
+
 // Plain epilogues: 4 consecutive columns n .. n + 3 of row m
 template <int EPI>
 __device__ __forceinline__ void store_out(const GemmParams& p, int m, int n, floatx4 v, floatx4 gv) {

@@ -49,11 +49,9 @@ __global__ __launch_bounds__(STHR, 1) void k_gemm16s(const GemmParams p) {
 
     const int i = (int)(blockIdx.x & 7) * p.per + (int)(blockIdx.x >> 3);  // XCD b % 8: a contiguous range of tiles
     if (i >= p.total) return;
-    constexpr int S_GROUP_M = 16;  // row tiles per raster group: consecutive workgroups share a weight tile in L2
-    const int per_group = S_GROUP_M * p.tiles_n;
-    const int g0 = (i / per_group) * S_GROUP_M;
-    const int gsz = min(S_GROUP_M, p.tiles_m - g0);
-    const int tm = g0 + (i % per_group) % gsz, tn = (i % per_group) / gsz;
+    constexpr int S_GROUP_M = 16;  // row tiles per raster group
+    int tm, tn;
+    raster_tile(i, S_GROUP_M, p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
     const int mrows = min(BM, p.M - m0);  // N is a multiple of BN
 
@@ -203,31 +201,7 @@ __global__ __launch_bounds__(STHR, 1) void k_gemm16s(const GemmParams p) {
     // the groups' sums meet in LDS; group kg finishes row blocks kg, kg + KG, ..
     constexpr int MBO = (MB + KG - 1) / KG;
     floatx4 out[NBW][MBO];
-    if constexpr (KG == 1) {
-#pragma unroll
-        for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) out[nb][mb] = acc[nb][mb];
-    } else {
-        floatx4* red = reinterpret_cast<floatx4*>(lds);
-        __syncthreads();  // every wave is done with the stages
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++) red[((wv * MB + mb) * NBW + nb) * 64 + lane] = acc[nb][mb];
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < MBO; j++) {
-            const int mb = min(kg + KG * j, MB - 1);
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++) {
-                floatx4 t = red[(((wv % (WN * WM)) * MB + mb) * NBW + nb) * 64 + lane];
-#pragma unroll
-                for (int k = 1; k < KG; k++) t += red[(((k * WN * WM + wv % (WN * WM)) * MB + mb) * NBW + nb) * 64 + lane];
-                out[nb][j] = t;
-            }
-        }
-    }
+    merge_k_groups<WN * WM, MB, KG>(acc, out, reinterpret_cast<floatx4*>(lds), wv, kg, lane);
     if constexpr (EPI == EPI_QKV) {
         qkv_epilogue<WN, WM, MB, KG, C::LDS / 2>(p, out, lds, m0, n0, wv, wn, wm, kg, lane);
     } else {

@@ -59,9 +59,9 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
     const int kg = wv / (WN * WM), wn = wv % (WN * WM) / WM, wm = wv % WM;
     const int i = (int)(blockIdx.x & 7) * p.per + (int)(blockIdx.x >> 3);  // XCD b % 8: a contiguous range of tiles
     if (i >= p.total) return;
-    constexpr int GROUP = 8;  // row tiles per raster group: consecutive workgroups share a weight tile in L2
-    const int per_group = GROUP * p.tiles_n, g0 = (i / per_group) * GROUP, gsz = min(GROUP, p.tiles_m - g0);
-    const int m0 = (g0 + (i % per_group) % gsz) * BM, n0 = (i % per_group) / gsz * BN;
+    int tm, tn;
+    raster_tile(i, 8, p.tiles_m, p.tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * BN;
     const int mrows = min(BM, p.T - m0), nrows = min(BN, p.rows - n0);
     const int KT = p.cols / 32, S = (KT + SL - 1) / SL;
 
@@ -188,31 +188,7 @@ __global__ __launch_bounds__(XTHR, 1) void k_linear_x3(const LinearParams p) {
 
     constexpr int MBO = (MB + KG - 1) / KG;
     floatx4 out[NBW][MBO];
-    if constexpr (KG == 1) {
-#pragma unroll
-        for (int nb = 0; nb < NBW; nb++)
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++) out[nb][mb] = acc[nb][mb];
-    } else {
-        floatx4* red = reinterpret_cast<floatx4*>(smem);
-        __syncthreads();  // every wave is done with the stages
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++) red[((wv * MB + mb) * NBW + nb) * 64 + lane] = acc[nb][mb];
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < MBO; j++) {
-            const int mb = min(kg + KG * j, MB - 1);
-#pragma unroll
-            for (int nb = 0; nb < NBW; nb++) {
-                floatx4 t = red[(((wv % (WN * WM)) * MB + mb) * NBW + nb) * 64 + lane];
-#pragma unroll
-                for (int k = 1; k < KG; k++) t += red[(((k * WN * WM + wv % (WN * WM)) * MB + mb) * NBW + nb) * 64 + lane];
-                out[nb][j] = t;
-            }
-        }
-    }
+    merge_k_groups<WN * WM, MB, KG>(acc, out, reinterpret_cast<floatx4*>(smem), wv, kg, lane);
 #pragma unroll
     for (int j = 0; j < MBO; j++) {
         const int mb = kg + KG * j, m = m0 + (wm * MB + mb) * 16 + rl;
