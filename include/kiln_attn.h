@@ -159,7 +159,9 @@ typedef enum { KILN_EPI_F32 = 0, KILN_EPI_F16 = 1, KILN_EPI_GELU16 = 2, KILN_EPI
  *   KILN_EPI_RESID:  y fp32 += gate[col] * acc   (gate fp32 [rows], NULL = 1)
  * y has rows of ldy >= rows elements. Requires rows % 128 == 0, cols % 32 == 0, k2 % 32 == 0 (the reference's
  * eligibility, tcgemm16.cuh:177) and 16-byte aligned x16/W/a2/w2 (KILN_EUNSUPPORTED otherwise, where the
- * reference throws); ldy even and y aligned to two elements. */
+ * reference throws); ldy even and y aligned to two elements. Repeated calls give the same bits. The order of a row's
+ * fp32 sum follows the workgroup tile, and the tile the sizes (kiln_linear16_tile): the same row in calls of different T
+ * may differ in its last bits. */
 int kiln_linear16(void* y, int ldy, const uint16_t* x16, int T, const uint16_t* w16, int rows, int cols, int epi,
                   const float* gate, float beta, const uint16_t* a2, const uint16_t* w2, int k2, kiln_stream_t stream);
 
@@ -209,7 +211,8 @@ int kiln_patchify(float* tok, const float* latent, int Hl, int Wl, kiln_stream_t
 int kiln_unpatchify(float* latent, const float* tok, int ldt, int Hl, int Wl, kiln_stream_t stream);
 /* Replaces linear() for the DiT's small fp32 layers (engine/src/gpu.h:118, kernels.cu:508-529; the x embedder
  * and the final layer, dit.cu:417,542): y [T, rows] (row stride ldy) = x [T, cols] (row stride ldx) W^T with
- * W bf16 [rows, cols], fp32 arithmetic. */
+ * W bf16 [rows, cols], fp32 arithmetic (products exact, sums fp32). Repeated calls give the same bits; the order of a
+ * row's sum follows the sizes, as for kiln_linear16. */
 int kiln_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols,
                     kiln_stream_t stream);
 /* Which kernel a kiln_linear_f32 call runs, for tests and profiles: the workgroup tile of the bf16 matrix-core form as

@@ -896,7 +896,10 @@ static hipError_t launch_sel(AttnParams p, int Tq, int units, hipStream_t s) {
     // spends most of a step waiting for its own chain of reads, exponentials and products (and, with 4 stages, for
     // the DMA issued one step earlier); the rows' arithmetic is the same. us per launch, H = 16, fp16 prepared Q, 32 rows
     // per wave -> 128-row units / 64-row units: T = 256 8.8 -> 7.7 / 6.7, 512 13.0 -> 11.4 / 9.8, 1024 21.8 -> 18.3 / 16.4,
-    // 1536 29.7 -> 26.1 / 40.4 (two rounds), 2048 40.4 -> 37.1; with two rounds of units 2304 52.0 -> 72.1
+    // 1536 29.7 -> 26.1 / 40.4 (two rounds), 2048 40.4 -> 37.1; with two rounds of units 2304 52.0 -> 72.1. Chains (two
+    // contexts and the NAG negative, the whole call), 4 waves x 32 rows -> 8 x 16, contexts of 23 / 141 / 512 / 1024 keys:
+    // T = 1536 20.3 / 25.9 / 41.1 / 62.6 -> 20.3 / 24.7 / 38.5 / 58.8, T = 2048 23.5 / 29.3 / 44.4 / 67.3 -> 23.0 / 28.1 /
+    // 45.3 / 67.3
     const long u64 = (long)((Tq + 63) / 64) * units, u128 = (long)((Tq + 127) / 128) * units;
     if (p.chain && u128 <= cus) return launch_nw<InT, OutT, QN, RP, 8, true, 1>(p, Tq, units, s);
     if (p.chain) return launch_nw<InT, OutT, QN, RP, 4, true>(p, Tq, units, s);

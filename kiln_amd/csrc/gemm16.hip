@@ -375,9 +375,10 @@ static int gemm16_mb(int M, int N, int cus, long* tiles) {
     return best;
 }
 
-// Few rows leave most CUs without a 256-wide tile: M = 256 x 2048 x 2048 takes 42.9 us on this kernel's 16 tiles
-// and 9.0 us on 64 x 32 ones, M = 1024 45.0 against 16.8 (128 x 64), M = 3072 49.3 against 35.5 (128 x 192); at
-// M = 4608 it is 54.0 against 72.5. The models meet near the size where the large tiles fill the chip.
+// Few rows leave most CUs without a 256-wide tile: M = 256 x 2048 x 2048 takes 47.1 us (39.5 with prepared weights) on this
+// kernel's 8 tiles and 9.9 on 64 x 32 ones, M = 1024 54.3 (44.4) against 17.5 (128 x 64), M = 3072 56.2 (48.0) against 33.6
+// (128 x 192); at M = 4608 it is 56.4 (47.3) against 58.8 (58.2). Weights from memory, fp16 out. The models meet near the
+// size where the large tiles fill the chip (gemm_cost gives both sides there).
 GemmTile gemm16_choose(int M, int N, int K, int epi) {
     const int cus = cu_count();
     long tiles = 0;

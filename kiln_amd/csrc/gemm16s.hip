@@ -11,10 +11,13 @@
 //    flight, with no partial sums in memory and a fixed order of summation.
 //  * a step's weights and activations stream global -> LDS by buffer-form DMA through NST stages of up to 48 KB,
 //    NST - 1 steps ahead; one barrier per step.
-//  * bound by the rate at which a CU takes in operand bytes (30 to 40 B per cycle in every configuration). Measured, us,
-//    one product of M rows with weights from memory, 256-wide tiles -> these: 2048 x 2048 M = 64 36.3 -> 9.3, M = 256
-//    42.9 -> 9.0, M = 1024 45.0 -> 16.7, M = 3072 47.8 -> 35.2; 2048 x 8192 M = 256 131.8 -> 25.3; 8192 x 2048 M = 256
-//    44.5 -> 19.0.
+//  * at M = 256 a CU takes in 40 (128 x 64) to 62 GB/s (64 x 32) of operands, a third to a half of what LDS DMA alone
+//    takes from L2 (120 to 130): what bounds these products is the chain of a step (barrier, operand reads, MFMAs) in the
+//    one workgroup of a CU, and where a product has fewer tiles than CUs (128 of 128 x 32 at 2048 x 2048, 192 of 128 x 64
+//    at 6144 x 2048), the idle ones. Measured, us, one product of M rows, fp16 out, weights from memory, 256-wide tiles with
+//    plain / prepared weights -> these (alike with both): 2048 x 2048 M = 64 44.6 / 35.6 -> 10.3, M = 256 47.1 / 39.5 -> 9.9,
+//    M = 1024 54.3 / 44.4 -> 17.5, M = 3072 56.2 / 48.0 -> 33.6; 2048 x 8192 M = 256 155.5 / 128.5 -> 25.7; 8192 x 2048
+//    M = 256 48.7 / 41.3 -> 18.9.
 //  * row-major operands (activations, plain weights) lie in LDS as 128-byte rows of two k slices, 16-byte chunk c
 //    of row r at position c ^ (r & 7): the DMA reads whole 128-byte lines, the operand reads are conflict free.
 //    Prepared weights keep their 64-byte rows (one contiguous run per slice).
@@ -268,9 +271,12 @@ hipError_t launch_gemm16s(const GemmParams& p, int cfg, int epi, hipStream_t s) 
 // the contention of the tiles in flight for L2 and HBM. The coefficients are least-squares fits of measured times
 // (M = 64 .. 6912 x {2048 x 2048, 8192 x 2048, 2048 x 8192, 6144 x 2048}, each configuration at every size, weights
 // rotated through memory), 10 to 18% off at most; the 128 x 128 tile's contention is set above its fit (0.055), where two
-// rounds of it meet the 256-wide tile (2048 x 8192, M = 4096 158 against 151). Over M = 512 .. 4608 of these products with
-// prepared weights the choice then costs at most 3% over the best one. It does not depend on the weight's layout, so a
-// prepared weight gives the bits of the row-major one.
+// rounds of it meet the 256-wide tile (2048 x 8192, M = 4096 158 against 151). It does not depend on the weight's layout,
+// so a prepared weight gives the bits of the row-major one, and where the two forms meet it is a compromise between the
+// layouts: 2048 x 2048, 256 x 224 tiles -> 128 x 128, fp16 / fp32 / residual out, M = 3584 plain 47.3 / 47.2 / 52.6 -> 43.2 /
+// 44.7 / 47.6, prepared 42.1 / 42.3 / 47.7 -> 41.9 / 43.8 / 47.7; M = 4096 plain 48.3 / 48.4 / 53.9 -> 44.2 / 46.5 / 50.4,
+// prepared 43.7 / 43.4 / 49.3 -> 43.3 / 45.5 / 50.5: at most 5% over the better one. A DiT block there: T = 3584 718 ->
+// 696, T = 4096 721 -> 727.
 double gemm_cost(const GemmCost& c, long tiles, int slices, int cus) {
     const double rounds = (double)((tiles + cus - 1) / cus);
     return c.launch + rounds * (c.tile + c.slice * slices) + c.shared * tiles * slices / cus;

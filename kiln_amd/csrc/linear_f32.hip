@@ -253,8 +253,8 @@ bool linear_x3_takes(const float* x, int ldx, const uint16_t* W, int T, int rows
 
 // The tile with the smallest modelled time (gemm_cost; fitted to measured times of every tile at T = 8 .. 6912 and the
 // DiT's widths, 6 to 12% off at most, its choice the measured best at all of them). us, v_mfma_f32_16x16x4_f32 ->
-// here: T = 120, 2048 x 1024 44.9 -> 9.3; T = 1024, 2048 x 2048 92.0 -> 30.6; T = 6912, 8192 x 2048 1840 -> 590 (393
-// TFLOP/s against the 154 of a large fp32 matrix product); T = 6912, 64 x 2048 61.2 -> 15.2. Error against 64 bits
+// here: T = 120, 2048 x 1024 44.9 -> 9.8; T = 1024, 2048 x 2048 92.0 -> 30.6; T = 6912, 8192 x 2048 1840 -> 560 (414
+// TFLOP/s against the 154 of a large fp32 matrix product); T = 6912, 64 x 2048 61.2 -> 16.4. Error against 64 bits
 // (2-norm, K = 2048): 8.1e-7 -> 1.7e-7 to 4.8e-7.
 LinearTile linear_x3_choose(int T, int rows, int cols) {
     static const struct {
