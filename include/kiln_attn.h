@@ -211,8 +211,8 @@ int kiln_patchify(float* tok, const float* latent, int Hl, int Wl, kiln_stream_t
 int kiln_unpatchify(float* latent, const float* tok, int ldt, int Hl, int Wl, kiln_stream_t stream);
 /* Replaces linear() for the DiT's small fp32 layers (engine/src/gpu.h:118, kernels.cu:508-529; the x embedder
  * and the final layer, dit.cu:417,542): y [T, rows] (row stride ldy) = x [T, cols] (row stride ldx) W^T with
- * W bf16 [rows, cols], fp32 arithmetic (products exact, sums fp32). Repeated calls give the same bits; the order of a
- * row's sum follows the sizes, as for kiln_linear16. */
+ * W bf16 [rows, cols], fp32 arithmetic: products exact, sums fp32 (weights below 2^-126, bf16's subnormals, count with
+ * 17 bits or more). Repeated calls give the same bits; the order of a row's sum follows the sizes, as for kiln_linear16. */
 int kiln_linear_f32(float* y, int ldy, const float* x, int ldx, const uint16_t* w_bf16, int T, int rows, int cols,
                     kiln_stream_t stream);
 /* Which kernel a kiln_linear_f32 call runs, for tests and profiles: the workgroup tile of the bf16 matrix-core form as
